@@ -1,0 +1,68 @@
+"""Closest-hit and any-hit traversal at the edges of the box test, against the oracle's brute force.
+
+The box test takes a plane's ray parameter as q * (step / d) + (origin - org) / d with a bound on
+the rounding of those two terms (kernels.hip, NodeAxis).  The cases here are the ones the bound
+is for: directions with zero, negative-zero and tiny components, unnormalised directions, origins
+on box planes and in the plane of flat triangles, and scenes far from the origin of coordinates,
+where the two terms cancel.  A culled box would lose a hit, so every hit must be the brute
+force's, bit for bit."""
+import numpy as np
+import pytest
+
+from oracle import binding as ob
+from tests.helpers import gpu_trace
+from vlr_amd import api, scenes
+
+pytestmark = pytest.mark.gpu
+
+INF = np.float32(3.4028235e38)
+
+
+def moved(desc, offset):
+    for inst in desc.instances:
+        inst.transform = inst.transform.copy()
+        inst.transform[12:15] += np.asarray(offset, np.float32)
+    return desc
+
+
+def edge_rays(kind, n, lo, hi, seed):
+    rng = np.random.default_rng(seed)
+    rays = np.zeros(n, api.RAY_DTYPE)
+    d = rng.normal(size=(n, 3))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    o = rng.uniform(lo, hi, size=(n, 3))
+    axis = rng.integers(0, 3, n)
+    if kind == "parallel":            # along an axis, the other components 0 or -0
+        s = rng.choice([-1.0, 1.0], n)
+        d = np.where(rng.random((n, 3)) < 0.5, 0.0, -0.0)
+        d[np.arange(n), axis] = s
+    elif kind == "one zero":
+        d[np.arange(n), axis] = rng.choice([0.0, -0.0], n)
+    elif kind == "tiny":
+        d[np.arange(n), axis] *= 10.0 ** -rng.uniform(6, 44, n)
+    elif kind == "unnormalised":
+        d *= 10.0 ** rng.uniform(-12, 12, (n, 1))
+    elif kind == "on planes":         # origins on the coordinates of the boxes' corners
+        o[np.arange(n), axis] = rng.choice([lo[1], hi[1], 0.0, 0.6, 1.2, 2.99], n)
+    rays["org"], rays["dir"], rays["tmax"] = o.astype(np.float32), d.astype(np.float32), INF
+    return rays
+
+
+@pytest.mark.parametrize("kind", ["parallel", "one zero", "tiny", "unnormalised", "on planes"])
+@pytest.mark.parametrize("scene,offset", [("cornell", 0.0), ("cornell", 3000.0), ("blobs", 0.0), ("blobs", 1000.0)])
+def test_edge_rays_hit_what_brute_force_hits(torch_gpu, kind, scene, offset):
+    desc = scenes.cornell_box() if scene == "cornell" else scenes.tessellated_cornell(3, 6000)
+    desc = moved(desc, (offset, -offset, 0.5 * offset))
+    c = np.array([offset, -offset, 0.5 * offset])
+    rays = edge_rays(kind, 4096 + 17, c + [-1.6, -0.1, -1.6], c + [1.6, 3.1, 1.6], 11)
+    with api.Context() as ctx:
+        bs = api.build_scene(ctx, desc)
+        hits = gpu_trace(torch_gpu, ctx, bs.scene, rays)
+        blocked = gpu_trace(torch_gpu, ctx, bs.scene, rays, any_hit=True)["inst"] >= 0
+    ref = ob.Scene(desc).trace_closest(rays, use_bvh=False)
+    found = ref["inst"] >= 0
+    print(kind, scene, offset, "hits", found.mean())
+    assert found.any()
+    np.testing.assert_array_equal(hits["inst"] >= 0, found)
+    np.testing.assert_array_equal(hits["t"][found], ref["t"][found])
+    np.testing.assert_array_equal(blocked, found)

@@ -28,6 +28,8 @@
 #include "launch.h"
 #include "radiance_cache.h"
 
+#include <type_traits>
+
 #pragma clang fp contract(off)
 
 // The build compiles this file once per unit (VLRA_UNIT): 1 RGB path tracing, 2 the same
@@ -66,7 +68,7 @@ namespace vlra {
 namespace VLRA_UNIT_NS {
 
 constexpr int kTraceBlock = 128;
-// per block: kLdsStack entries per lane of node codes, then as many entry distances
+// per block: kLdsStack entries per lane, a node code and an entry distance each
 constexpr int kTraceLds = 2 * kLdsStack * kTraceBlock;
 // A CU's 160 KB of LDS holds 9 blocks of kTraceLds (4.5 waves per SIMD).  The per-depth
 // closest-hit kernel keeps 12 entries per lane (12 KB per block), so that its registers (5 waves
@@ -91,39 +93,71 @@ constexpr int32_t kSentinel = INT32_MIN;
 
 // ---------------------------------------------------------------------------------------------
 // ray set-up and primitive tests
+//
+// Box tests.  A child plane is the grid value o + q * s (q a byte, s a power of two), so the ray
+// parameter at it is q * (s * inv) + (o - org) * inv: one conversion and one fused multiply-add per
+// plane, with the node's six constants computed once for its four children, where decoding the
+// plane first (q * s, + o, - org, * inv) takes five operations.  The sign of the direction selects
+// which of the two planes is the near one for all four children at once, in place of a minimum and
+// a maximum per child and axis.  The traversal is bound by VALU issue (k_tail: 0.62 of one
+// instruction per CU and cycle at 19 % of its lanes), so operations count: against decoded planes,
+// generic stack pointers (flat accesses) and per-child branches, a 256 x 256 Cornell frame went from
+// 0.52 to 0.30 ms, the 1080p icosphere grid's from 3.9 to 3.4 ms, 2^21 incoherent closest-hit rays
+// in that grid from 2.14 to 1.80 ms.
+//   The constants cancel (o - org against q * s), so their rounding is bounded absolutely.  With
+// u = 2^-24, a = s * inv, b = fma(o, inv, -org * inv) and M = |org inv| + |b| + 256 |a|, a computed
+// plane parameter is off by: the plane as stored (the builder's check rounds o + q * s once), at
+// most u M; the rounding of org * inv, of b, of the widened constant and of the multiply-add, at
+// most u M each in the terms they hold; the reciprocal's one ulp, 2 u (|b| + 256 |a|).  That is
+// less than 8 u M in all, and the near constant is lowered and the far one raised by 2^-21 M: no
+// box is culled that holds a hit the triangle test would report.
 struct RayPre {
-    V3 org, dir, inv;
-    int kx, ky, kz;
+    V3 org, inv, oi;          // oi = org * inv
+    int kz;                   // axis of the largest direction component
     float Sx, Sy, Sz;
     __device__ __forceinline__ void init(const V3 &o, const V3 &d) {
         org = o;
-        dir = d;
         kz = 0;
-        float adx = fabsf(d.x), ady = fabsf(d.y), adz = fabsf(d.z);
+        const float adx = fabsf(d.x), ady = fabsf(d.y), adz = fabsf(d.z);
         float best = adx;
         if (ady > best) { kz = 1; best = ady; }
-        if (adz > best) { kz = 2; }
-        kx = kz == 2 ? 0 : kz + 1;
-        ky = kx == 2 ? 0 : kx + 1;
-        float dkz = d[kz];
-        if (dkz < 0.0f) { int t = kx; kx = ky; ky = t; }
-        Sx = d[kx] / dkz;
-        Sy = d[ky] / dkz;
+        if (adz > best) { kz = 2; best = adz; }
+        // The triangle test's shear along kz, in the cyclic order kz, kz + 1, kz + 2.  (Exchanging
+        // the last two for a negative direction only negates U, V, W and the determinant together,
+        // which leaves every tested sign relation and every result bit the same.)
+        const float dkz = rot0(d);
+        Sx = rot1(d) / dkz;
+        Sy = rot2(d) / dkz;
         Sz = 1.0f / dkz;
-        inv = V3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+        // Directions of a component below 2^-60 of the largest count as that: the planes' parameters
+        // stay finite, and no point of the ray moves by more than 2^-60 of its distance.
+        const float tiny = fmaxf(best * 8.6736174e-19f, 1.17549435e-38f);
+        inv.x = __builtin_amdgcn_rcpf(copysignf(fmaxf(adx, tiny), d.x));
+        inv.y = __builtin_amdgcn_rcpf(copysignf(fmaxf(ady, tiny), d.y));
+        inv.z = __builtin_amdgcn_rcpf(copysignf(fmaxf(adz, tiny), d.z));
+        oi = V3(o.x * inv.x, o.y * inv.y, o.z * inv.z);
+    }
+    // component kz, kz + 1, kz + 2 (cyclic) of v
+    __device__ __forceinline__ float rot0(const V3 &v) const { return pick(v.x, v.y, v.z); }
+    __device__ __forceinline__ float rot1(const V3 &v) const { return pick(v.y, v.z, v.x); }
+    __device__ __forceinline__ float rot2(const V3 &v) const { return pick(v.z, v.x, v.y); }
+    __device__ __forceinline__ float pick(float k0, float k1, float k2) const {
+        float r = kz == 1 ? k1 : k0;
+        r = kz == 2 ? k2 : r;
+        return r;
     }
 };
 
 __device__ __forceinline__ bool intersectTri(const RayPre &r, const V3 &p0, const V3 &p1, const V3 &p2, float tmin,
                                              float tmax, float *tOut, float *b1Out, float *b2Out) {
     const V3 A = p0 - r.org, B = p1 - r.org, C = p2 - r.org;
-    const float Akz = A[r.kz], Bkz = B[r.kz], Ckz = C[r.kz];
-    const float Ax = A[r.kx] - r.Sx * Akz;
-    const float Ay = A[r.ky] - r.Sy * Akz;
-    const float Bx = B[r.kx] - r.Sx * Bkz;
-    const float By = B[r.ky] - r.Sy * Bkz;
-    const float Cx = C[r.kx] - r.Sx * Ckz;
-    const float Cy = C[r.ky] - r.Sy * Ckz;
+    const float Akz = r.rot0(A), Bkz = r.rot0(B), Ckz = r.rot0(C);
+    const float Ax = r.rot1(A) - r.Sx * Akz;
+    const float Ay = r.rot2(A) - r.Sy * Akz;
+    const float Bx = r.rot1(B) - r.Sx * Bkz;
+    const float By = r.rot2(B) - r.Sy * Bkz;
+    const float Cx = r.rot1(C) - r.Sx * Ckz;
+    const float Cy = r.rot2(C) - r.Sy * Ckz;
     float U = Cx * By - Cy * Bx;
     float V = Ax * Cy - Ay * Cx;
     float W = Bx * Ay - By * Ax;
@@ -145,19 +179,18 @@ __device__ __forceinline__ bool intersectTri(const RayPre &r, const V3 &p0, cons
     return true;
 }
 
-// Conservative slab test: the exit distance is widened by a few ulps so rounding never culls
-// a box that holds a hit the triangle test would report.
-__device__ __forceinline__ bool slab(const V3 &lo, const V3 &hi, const RayPre &r, float tmin, float tmax,
-                                     float *tEnter) {
-    float tx0 = (lo.x - r.org.x) * r.inv.x, tx1 = (hi.x - r.org.x) * r.inv.x;
-    float ty0 = (lo.y - r.org.y) * r.inv.y, ty1 = (hi.y - r.org.y) * r.inv.y;
-    float tz0 = (lo.z - r.org.z) * r.inv.z, tz1 = (hi.z - r.org.z) * r.inv.z;
-    float tn = fmaxf(fmaxf(fminf(tx0, tx1), fminf(ty0, ty1)), fmaxf(fminf(tz0, tz1), tmin));
-    float tf = fminf(fminf(fmaxf(tx0, tx1), fmaxf(ty0, ty1)), fmaxf(tz0, tz1));
-    tf = fminf(tf * (1.0f + 8.0f * __FLT_EPSILON__), tmax * (1.0f + 8.0f * __FLT_EPSILON__));
-    *tEnter = tn;
-    return tn <= tf;
-}
+// One axis of a node against a ray: plane parameters are fma(q, a, bNear / bFar).
+struct NodeAxis {
+    float a, bNear, bFar;
+    __device__ __forceinline__ NodeAxis(float origin, float step, float inv, float oi) {
+        a = step * inv;
+        const float b = __builtin_fmaf(origin, inv, -oi);
+        const float e = __builtin_fmaf(fabsf(oi), 4.7683716e-7f,
+                                       __builtin_fmaf(fabsf(b), 4.7683716e-7f, fabsf(a) * 1.2207031e-4f));
+        bNear = b - e;
+        bFar = b + e;
+    }
+};
 
 struct TraceHit {
     int32_t inst, geomInst, prim;
@@ -170,16 +203,20 @@ struct TravCount {
     uint32_t nodes = 0, tris = 0, insts = 0;
 };
 
+typedef int32_t StackPair __attribute__((ext_vector_type(2)));   // node code, entry distance
+
 // Traversal state: one ray's walk through the two-level BVH.  The node stack
 // lives in LDS (kLdsStack entries per lane) with an overflow area the caller keeps in scratch.
 constexpr int32_t kTravDone = INT32_MIN + 1;
 struct TravState {
-    RayPre world, ray;
+    V3 org, dir;                  // the world-space ray
+    RayPre ray;                   // in the space of the tree being walked
     float tmin, tmax;
     int32_t cur, curInst;
-    int sp;
-    uint32_t blasNode, blasTri;   // bases of the instance being traversed
-    bool inBlas, found, anyHit;
+    int sp, spBlas;               // stack height, and the height at which the instance was entered
+    const BVH4QNode *nodes;       // the tree being walked
+    const TriRecord *tris;
+    bool inBlas, found;
     TraceHit hit;
     Pcg32 *rng;                   // the path's generator for the stochastic alpha test
     float vis;                    // fractional visibility of an any-hit ray through alpha surfaces
@@ -190,18 +227,19 @@ __device__ __forceinline__ float alphaAt(const DevScene &sc, int32_t inst, uint3
                                          float b2);
 
 __device__ __forceinline__ void travBegin(TravState &st, const DevScene &sc, const V3 &org, const V3 &dir, float tmin,
-                                          float tmax, bool anyHit) {
-    st.world.init(org, dir);
-    st.ray = st.world;
+                                          float tmax) {
+    st.org = org;
+    st.dir = dir;
+    st.ray.init(org, dir);
     st.tmin = tmin;
     st.tmax = tmax;
     st.cur = sc.hasTlas ? 0 : kTravDone;
     st.curInst = -1;
-    st.sp = 0;
-    st.blasNode = st.blasTri = 0;
+    st.sp = st.spBlas = 0;
+    st.nodes = sc.tlasNodes;
+    st.tris = sc.blasTris;
     st.inBlas = false;
     st.found = false;
-    st.anyHit = anyHit;
     st.hit.inst = -1;
     st.hit.geomInst = st.hit.prim = -1;
     st.hit.t = st.hit.b1 = st.hit.b2 = 0.0f;
@@ -211,7 +249,7 @@ __device__ __forceinline__ void travBegin(TravState &st, const DevScene &sc, con
 
 // Runs the traversal to its end (then st.found and st.hit hold the closest hit, or any hit for
 // an any-hit ray).  The loop is a while-while loop: a lane walks inner nodes until it reaches a
-// leaf, an instance's end marker or the end of the walk, and only then handles that one item
+// leaf, an instance's end or the end of the walk, and only then handles that one item
 // (enter the instance, test the leaf's triangles, or leave the instance) before walking inner
 // nodes again.  Each lane visits the same nodes in the same order as a one-item-per-iteration
 // loop; the wave just runs its lanes' inner-node visits together and their leaves together.
@@ -220,145 +258,136 @@ __device__ __forceinline__ void travBegin(TravState &st, const DevScene &sc, con
 // (light_transport_common.h:205-218) for any-hit rays.
 // ANY: an any-hit ray, which needs no visiting order: its children are stacked as they come,
 // without entry distances.
-// SD: stack entries per lane in LDS (lds holds SD * kTraceBlock node codes, then as many entry
-// distances unless ANY); the other kTravStackCapacity - SD entries are in ovf / ovfT.
-template <bool ANY, bool STATS, bool ALPHA = false, int SD = kLdsStack>
-__device__ __forceinline__ void traverse(TravState &st, const DevScene &sc, int32_t *lds, int lane, int32_t *ovf,
-                                         float *ovfT, TravCount *tc) {
+// SD: stack entries per lane in LDS, (code, entry distance) pairs of which an any-hit ray uses the
+// codes; the other kTravStackCapacity - SD entries are in ovf.  A lane's entries have the same
+// places for both kinds of rays, because the waves of a block run the two at the same time.  CODES:
+// places for codes only, in a kernel that traces nothing but any-hit rays.
+template <bool ANY, bool STATS, bool ALPHA = false, int SD = kLdsStack, bool CODES = false>
+__device__ __forceinline__ void traverse(TravState &st, const DevScene &sc, int32_t *ldsWords, int lane,
+                                         TravCount *tc) {
     constexpr int kOvf = static_cast<int>(kTravStackCapacity) - SD;
-    float *ldsT = ANY ? nullptr : reinterpret_cast<float *>(lds + SD * kTraceBlock);
     // each stack entry keeps the distance at which the ray enters its box; once a closer hit
-    // has shrunk tmax past it (with the slab test's widening), the entry is dropped unvisited.
+    // has shrunk tmax past it (widened by 8 ulps), the entry is dropped unvisited.
     // Scene set-up bounds the depth by kTravStackCapacity (travStackBound), so the index never
     // reaches past the scratch area; the clamp only keeps the access inside the array.
-    auto push = [&](int32_t v, float tEnter) {
-        if (st.sp < SD) {
-            lds[st.sp * kTraceBlock + lane] = v;
-            if constexpr (!ANY) ldsT[st.sp * kTraceBlock + lane] = tEnter;
-        } else {
-            ovf[min(st.sp - SD, kOvf - 1)] = v;
-            if constexpr (!ANY) ovfT[min(st.sp - SD, kOvf - 1)] = tEnter;
-        }
-        ++st.sp;
+    // The LDS part is addressed as LDS: with generic pointers the two parts' accesses merge into
+    // flat ones, which wait for every memory counter.
+    using Entry = std::conditional_t<ANY, int32_t, StackPair>;
+    static_assert(ANY || !CODES, "closest-hit rays keep entry distances");
+    constexpr int kStride = kTraceBlock * (ANY && !CODES ? 2 : 1);   // from one entry of a lane to the next
+    auto *lds = (__attribute__((address_space(3))) Entry *)ldsWords + lane * (kStride / kTraceBlock);
+    Entry ovf[kOvf];
+    auto entry = [](int32_t v, float t) -> Entry {
+        if constexpr (ANY) return v;
+        else return StackPair{v, __float_as_int(t)};
+    };
+    auto store = [&](int at, int32_t v, float t) {
+        if (at < SD) lds[at * kStride] = entry(v, t);
+        else ovf[min(at - SD, kOvf - 1)] = entry(v, t);
     };
     // pop, dropping entries that lie beyond the closest hit so far (an any-hit ray stops at its
-    // first hit, so every entry it pops is still open)
+    // first hit, so every entry it pops is still open); kSentinel when the instance's part of the
+    // stack is used up, kTravDone when all of it is
     auto pop = [&]() -> int32_t {
-        if constexpr (ANY) {
-            if (st.sp == 0) return kTravDone;
+        const int base = st.inBlas ? st.spBlas : 0;
+        const float tCull = st.tmax * (1.0f + 8.0f * __FLT_EPSILON__);
+        while (st.sp > base) {
             --st.sp;
-            return st.sp < SD ? lds[st.sp * kTraceBlock + lane] : ovf[min(st.sp - SD, kOvf - 1)];
-        } else {
-            const float tCull = st.tmax * (1.0f + 8.0f * __FLT_EPSILON__);
-            while (st.sp > 0) {
-                --st.sp;
-                float te;
-                int32_t v;
-                if (st.sp < SD) {
-                    v = lds[st.sp * kTraceBlock + lane];
-                    te = ldsT[st.sp * kTraceBlock + lane];
-                } else {
-                    v = ovf[min(st.sp - SD, kOvf - 1)];
-                    te = ovfT[min(st.sp - SD, kOvf - 1)];
-                }
-                if (te <= tCull) return v;
-            }
-            return kTravDone;
+            Entry e;
+            if (st.sp < SD) e = lds[st.sp * kStride];
+            else e = ovf[min(st.sp - SD, kOvf - 1)];
+            if constexpr (ANY) return e;
+            else if (__int_as_float(e.y) <= tCull) return e.x;
         }
+        return st.inBlas ? kSentinel : kTravDone;
     };
     while (st.cur != kTravDone) {
         // inner nodes
         while (st.cur >= 0) {
-            const int32_t cur = st.cur;
             if constexpr (STATS) ++tc->nodes;
-            const BVH4QNode *nodes = st.inBlas ? sc.blasNodes + st.blasNode : sc.tlasNodes;
-            const uint4 *np = reinterpret_cast<const uint4 *>(nodes + cur);
-            const uint4 w0 = np[0], w1 = np[1], w2 = np[2], w3 = np[3];
-            // decode: origin + q * step per axis (step = 2^(e - 127), exact product)
-            const float ox = __uint_as_float(w0.x), oy = __uint_as_float(w0.y), oz = __uint_as_float(w0.z);
-            const float sx = __uint_as_float((w0.w & 0xFFu) << 23), sy = __uint_as_float(((w0.w >> 8) & 0xFFu) << 23),
-                        sz = __uint_as_float(((w0.w >> 16) & 0xFFu) << 23);
-            const uint32_t qlx = w1.x, qly = w1.y, qlz = w1.z, qhx = w1.w, qhy = w2.x, qhz = w2.y;
-            auto lo = [&](int k) {
-                return V3(ox + static_cast<float>((qlx >> (8 * k)) & 0xFFu) * sx,
-                          oy + static_cast<float>((qly >> (8 * k)) & 0xFFu) * sy,
-                          oz + static_cast<float>((qlz >> (8 * k)) & 0xFFu) * sz);
-            };
-            auto hi = [&](int k) {
-                return V3(ox + static_cast<float>((qhx >> (8 * k)) & 0xFFu) * sx,
-                          oy + static_cast<float>((qhy >> (8 * k)) & 0xFFu) * sy,
-                          oz + static_cast<float>((qhz >> (8 * k)) & 0xFFu) * sz);
-            };
-            // child code 0 (the root's index) marks an empty slot
+            const uint4 *np = reinterpret_cast<const uint4 *>(st.nodes + st.cur);
+            const uint4 w0 = np[0], w1 = np[1], w2 = np[2];
+            const uint2 w3 = *reinterpret_cast<const uint2 *>(np + 3);
+            const RayPre &r = st.ray;
+            // step = 2^(e - 127) per axis
+            const NodeAxis X(__uint_as_float(w0.x), __uint_as_float((w0.w << 23) & 0x7F800000u), r.inv.x, r.oi.x),
+                Y(__uint_as_float(w0.y), __uint_as_float((w0.w << 15) & 0x7F800000u), r.inv.y, r.oi.y),
+                Z(__uint_as_float(w0.z), __uint_as_float((w0.w << 7) & 0x7F800000u), r.inv.z, r.oi.z);
+            const bool nx = r.inv.x < 0.0f, ny = r.inv.y < 0.0f, nz = r.inv.z < 0.0f;
+            const uint32_t qnx = nx ? w1.w : w1.x, qfx = nx ? w1.x : w1.w;
+            const uint32_t qny = ny ? w2.x : w1.y, qfy = ny ? w1.y : w2.x;
+            const uint32_t qnz = nz ? w2.y : w1.z, qfz = nz ? w1.z : w2.y;
+            const float tmaxWide = st.tmax * (1.0f + 8.0f * __FLT_EPSILON__);
             constexpr float kMiss = __builtin_huge_valf();
-            float t0 = kMiss, t1 = kMiss, t2 = kMiss, t3 = kMiss;
+            // entry distance of child k, or kMiss; child code 0 (the root's index) marks an empty slot
+            auto enter = [&](int k, int32_t c) {
+                auto q = [&](uint32_t w) { return static_cast<float>((w >> (8 * k)) & 0xFFu); };
+                const float tn = fmaxf(fmaxf(fmaxf(__builtin_fmaf(q(qnx), X.a, X.bNear), __builtin_fmaf(q(qny), Y.a, Y.bNear)),
+                                             __builtin_fmaf(q(qnz), Z.a, Z.bNear)), st.tmin);
+                const float tf = fminf(fminf(__builtin_fmaf(q(qfx), X.a, X.bFar), __builtin_fmaf(q(qfy), Y.a, Y.bFar)),
+                                       __builtin_fmaf(q(qfz), Z.a, Z.bFar));
+                return (c != 0) & (tn <= fminf(tf, tmaxWide)) ? tn : kMiss;
+            };
             int32_t c0 = static_cast<int32_t>(w2.z), c1 = static_cast<int32_t>(w2.w), c2 = static_cast<int32_t>(w3.x),
                     c3 = static_cast<int32_t>(w3.y);
-            float tt;
-            if (c0 != 0 && slab(lo(0), hi(0), st.ray, st.tmin, st.tmax, &tt)) t0 = tt;
-            if (c1 != 0 && slab(lo(1), hi(1), st.ray, st.tmin, st.tmax, &tt)) t1 = tt;
-            if (c2 != 0 && slab(lo(2), hi(2), st.ray, st.tmin, st.tmax, &tt)) t2 = tt;
-            if (c3 != 0 && slab(lo(3), hi(3), st.ray, st.tmin, st.tmax, &tt)) t3 = tt;
-            const int hits = (t0 != kMiss) + (t1 != kMiss) + (t2 != kMiss) + (t3 != kMiss);
-            if (ANY && hits > 0) {
+            float t0 = enter(0, c0), t1 = enter(1, c1), t2 = enter(2, c2), t3 = enter(3, c3);
+            if constexpr (ANY) {
                 // any order will do: stack the hit children but the first, visit that one next
                 int32_t next = 0;   // 0 is never a child code
                 auto take = [&](int32_t c, float t) {
-                    if (t == kMiss) return;
-                    if (next == 0) next = c;
-                    else push(c, t);
+                    const bool hit = t != kMiss, more = hit && next != 0;
+                    if (more) store(st.sp, c, t);
+                    st.sp += more;
+                    next = hit && next == 0 ? c : next;
                 };
                 take(c0, t0);
                 take(c1, t1);
                 take(c2, t2);
                 take(c3, t3);
                 st.cur = next;
-            } else if (hits > 0) {
+                if (next == 0) st.cur = pop();
+            } else {
                 // sort the four (distance, child) pairs, nearest first; misses sort last
                 auto cswap = [](float &ta, int32_t &ca, float &tb, int32_t &cb) {
-                    if (tb < ta) {
-                        float t = ta; ta = tb; tb = t;
-                        int32_t c = ca; ca = cb; cb = c;
-                    }
+                    const bool s = tb < ta;
+                    const float tl = s ? tb : ta, th = s ? ta : tb;
+                    const int32_t cl = s ? cb : ca, ch = s ? ca : cb;
+                    ta = tl; tb = th;
+                    ca = cl; cb = ch;
                 };
                 cswap(t0, c0, t1, c1);
                 cswap(t2, c2, t3, c3);
                 cswap(t0, c0, t2, c2);
                 cswap(t1, c1, t3, c3);
                 cswap(t1, c1, t2, c2);
-                if (hits > 3) push(c3, t3);
-                if (hits > 2) push(c2, t2);
-                if (hits > 1) push(c1, t1);
+                if (st.sp + 3 <= SD) {
+                    // the entries go to consecutive places, a miss being overwritten by the next
+                    auto *top = lds + st.sp * kStride;
+                    top[0] = entry(c3, t3);
+                    top += t3 != kMiss ? kStride : 0;
+                    st.sp += t3 != kMiss;
+                    top[0] = entry(c2, t2);
+                    top += t2 != kMiss ? kStride : 0;
+                    st.sp += t2 != kMiss;
+                    top[0] = entry(c1, t1);
+                    st.sp += t1 != kMiss;
+                } else {
+                    if (t3 != kMiss) store(st.sp++, c3, t3);
+                    if (t2 != kMiss) store(st.sp++, c2, t2);
+                    if (t1 != kMiss) store(st.sp++, c1, t1);
+                }
                 st.cur = c0;
-            } else {
-                st.cur = pop();
+                if (t0 == kMiss) st.cur = pop();
             }
         }
         if (st.cur == kTravDone) break;
-        const int32_t cur = st.cur;
-        if (cur != kSentinel) {
-            const uint32_t code = ~static_cast<uint32_t>(cur);
+        if (st.inBlas && st.cur != kSentinel) {
+            const uint32_t code = ~static_cast<uint32_t>(st.cur);
             const uint32_t first = code >> kLeafShift;
             const uint32_t count = (code & (kMaxLeafPrims - 1)) + 1;
-            if (!st.inBlas) {
-                // enter the instance: object-space ray, BLAS root, return marker on the stack
-                if constexpr (STATS) ++tc->insts;
-                const DevInstance &I = sc.instances[first];
-                V3 o = xfmPoint(I.w2o, st.world.org);
-                V3 d = xfmVector(I.w2o, st.world.dir);
-                st.ray.init(o, d);
-                st.curInst = static_cast<int32_t>(first);
-                st.blasNode = I.blasNodeBase;
-                st.blasTri = I.blasTriBase;
-                st.inBlas = true;
-                push(kSentinel, -__builtin_huge_valf());
-                st.cur = 0;
-                continue;
-            }
             if constexpr (STATS) tc->tris += count;
-            const TriRecord *tris = sc.blasTris + st.blasTri;
             for (uint32_t k = 0; k < count; ++k) {
-                const float4 *tp = reinterpret_cast<const float4 *>(tris + first + k);
+                const float4 *tp = reinterpret_cast<const float4 *>(st.tris + first + k);
                 const float4 q0 = tp[0], q1 = tp[1], q2 = tp[2];
                 float t, b1, b2;
                 if (intersectTri(st.ray, xyz(q0), xyz(q1), xyz(q2), st.tmin, st.tmax, &t, &b1, &b2)) {
@@ -389,27 +418,45 @@ __device__ __forceinline__ void traverse(TravState &st, const DevScene &sc, int3
                 st.cur = kTravDone;
                 break;
             }
-        } else {
-            // leave the instance
-            st.inBlas = false;
-            st.ray = st.world;
+            st.cur = pop();
+            continue;
         }
-        st.cur = pop();
+        // Leave the instance (kSentinel), enter the next one (a leaf of the top-level tree), or
+        // both: the ray is set up once for the space the walk goes on in.
+        if (st.cur == kSentinel) {
+            st.inBlas = false;
+            st.cur = pop();
+            if (st.cur == kTravDone) break;
+        }
+        V3 o = st.org, d = st.dir;
+        if (st.cur < 0) {
+            if constexpr (STATS) ++tc->insts;
+            st.curInst = static_cast<int32_t>((~static_cast<uint32_t>(st.cur)) >> kLeafShift);
+            const DevInstance &I = sc.instances[st.curInst];
+            o = xfmPoint(I.w2o, st.org);
+            d = xfmVector(I.w2o, st.dir);
+            st.nodes = sc.blasNodes + I.blasNodeBase;
+            st.tris = sc.blasTris + I.blasTriBase;
+            st.inBlas = true;
+            st.spBlas = st.sp;
+            st.cur = 0;
+        } else {
+            st.nodes = sc.tlasNodes;
+        }
+        st.ray.init(o, d);
     }
 }
 
 // rng: the path's generator (closest-hit rays through alpha surfaces); vis: the fractional
 // visibility of an any-hit ray (0 when occluded)
-template <bool ANY, bool STATS = false, bool ALPHA = false, int SD = kLdsStack>
+template <bool ANY, bool STATS = false, bool ALPHA = false, int SD = kLdsStack, bool CODES = false>
 __device__ __forceinline__ bool traceRay(const DevScene &sc, const V3 &org, const V3 &dir, float tmin, float tmax,
                                          TraceHit *hit, int32_t *lds, int lane, TravCount *tc = nullptr,
                                          Pcg32 *rng = nullptr, float *vis = nullptr) {
     TravState st;
-    travBegin(st, sc, org, dir, tmin, tmax, ANY);
+    travBegin(st, sc, org, dir, tmin, tmax);
     st.rng = rng;
-    int32_t ovf[kTravStackCapacity - SD];
-    float ovfT[ANY ? 1 : kTravStackCapacity - SD];
-    traverse<ANY, STATS, ALPHA, SD>(st, sc, lds, lane, ovf, ovfT, tc);
+    traverse<ANY, STATS, ALPHA, SD, CODES>(st, sc, lds, lane, tc);
     if (st.found) *hit = st.hit;
     if (vis) *vis = st.found ? 0.0f : st.vis;
     return st.found;
@@ -936,7 +983,7 @@ __device__ __forceinline__ void addTravStats(uint32_t *counters, uint32_t slot, 
 // ---- intersect: closest hit ----
 template <bool STATS, bool MULTI = false, bool ALPHA = false>
 __global__ void __launch_bounds__(kTraceBlock) k_intersect(KArgs a) {
-    __shared__ int32_t lds[kIntersectLds];
+    __shared__ __attribute__((aligned(8))) int32_t lds[kIntersectLds];
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     const RayQueue q = a.fb.rays[a.depth & 1];
     const uint32_t count = a.fb.counters[2 * a.depth];
@@ -1370,7 +1417,7 @@ __device__ __forceinline__ void firstHitGuides(const KArgs &a, uint32_t path, co
 // tests draw from the same generator), whose guides are added.
 template <int N, bool NODES>
 __global__ void __launch_bounds__(kTraceBlock) k_ltGuides(KArgs a) {
-    __shared__ int32_t lds[kTraceLds];
+    __shared__ __attribute__((aligned(8))) int32_t lds[kTraceLds];
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= a.fp.imageW * a.fp.imageH) return;
     const uint32_t px = i % a.fp.imageW, py = i / a.fp.imageW;
@@ -1440,7 +1487,7 @@ __global__ void __launch_bounds__(256) k_shade(KArgs a) {
 // ---- shadow: any-hit, adds the NEE contribution when unoccluded ----
 template <bool STATS, bool MULTI = false, bool ALPHA = false>
 __global__ void __launch_bounds__(kTraceBlock) k_shadow(KArgs a) {
-    __shared__ int32_t lds[kShadowLds];
+    __shared__ __attribute__((aligned(8))) int32_t lds[kShadowLds];
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t count = a.fb.counters[2 * a.depth + 1];
     TravCount tc;
@@ -1450,11 +1497,11 @@ __global__ void __launch_bounds__(kTraceBlock) k_shadow(KArgs a) {
         bool occluded;
         float vis = 1.0f;
         if constexpr (MULTI)
-            occluded = traceRay<true, STATS>(a.jobs[jobOf(a, __float_as_uint(o.w))].scene, xyz(o), xyz(d), 0.0f,
+            occluded = traceRay<true, STATS, false, kLdsStack, true>(a.jobs[jobOf(a, __float_as_uint(o.w))].scene, xyz(o), xyz(d), 0.0f,
                                              d.w, &h, lds, threadIdx.x, &tc);
         else
-            occluded = traceRay<true, STATS, ALPHA>(a.sc, xyz(o), xyz(d), 0.0f, d.w, &h, lds, threadIdx.x, &tc,
-                                                    nullptr, &vis);
+            occluded = traceRay<true, STATS, ALPHA, kLdsStack, true>(a.sc, xyz(o), xyz(d), 0.0f, d.w, &h, lds,
+                                                                      threadIdx.x, &tc, nullptr, &vis);
         if (!occluded) {
             uint32_t path = __float_as_uint(o.w);
             float4 v = a.fb.shadow.value[i];
@@ -1476,7 +1523,7 @@ __global__ void __launch_bounds__(kTraceBlock) k_shadow(KArgs a) {
 template <int N, bool STATS, bool MULTI = false, bool NODES = true>
 __global__ void __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(kTailWavesPerEU)))
 k_tail(KArgs a) {
-    __shared__ int32_t lds[kTraceLds];
+    __shared__ __attribute__((aligned(8))) int32_t lds[kTraceLds];
     __shared__ uint32_t depthCounts[2 * kMaxDepthCounters];
     const DevScene &sc = a.sc;
     const uint32_t depth0 = a.depth;
@@ -2055,7 +2102,7 @@ __device__ __forceinline__ Wls<N> commonWls(const BptParams &bp, bool single) {
 template <int N, bool NODES = true>
 __global__ void __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(kBptLightWavesPerEU)))
 k_bptLight(BptArgs a) {
-    __shared__ int32_t lds[kTraceLds];
+    __shared__ __attribute__((aligned(8))) int32_t lds[kTraceLds];
     const DevScene &sc = a.sc;
     const BptParams &bp = a.bp;
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2283,7 +2330,7 @@ __global__ void __launch_bounds__(256) k_bptCompact(BptParams bp) {
 template <int N, bool NODES = true, bool GUIDES = false>
 __global__ void __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(kBptEyeWavesPerEU)))
 k_bptEye(BptArgs a) {
-    __shared__ int32_t lds[kTraceLds];
+    __shared__ __attribute__((aligned(8))) int32_t lds[kTraceLds];
     const DevScene &sc = a.sc;
     const BptParams &bp = a.bp;
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2677,7 +2724,7 @@ __device__ __forceinline__ void sampleLens(const DevCamera &cam, float ul0, floa
 template <int N, bool NODES = true>
 __global__ void __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(kLightTraceWavesPerEU)))
 k_lightTrace(BptArgs a) {
-    __shared__ int32_t lds[kTraceLds];
+    __shared__ __attribute__((aligned(8))) int32_t lds[kTraceLds];
     const DevScene &sc = a.sc;
     const BptParams &bp = a.bp;
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2895,7 +2942,7 @@ struct HitOut { int32_t inst, geomInst, prim; float t, b1, b2; };
 
 template <bool ANY>
 __global__ void __launch_bounds__(kTraceBlock) k_traceRays(DevScene sc, const RayIn *rays, uint32_t n, HitOut *hits) {
-    __shared__ int32_t lds[kTraceLds];
+    __shared__ __attribute__((aligned(8))) int32_t lds[kTraceLds];
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     RayIn r = rays[i];
