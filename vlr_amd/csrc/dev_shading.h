@@ -70,30 +70,43 @@ struct Spec {
         for (int i = 0; i < N; ++i) f = f && isfinite(v[i]);
         return f;
     }
-    __device__ __forceinline__ float importance(uint32_t sel) const {
-        float sum = 0;
-        float picked = v[0];
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-            sum += v[i];
-            if (i == static_cast<int>(sel)) picked = v[i];
-        }
-        const float primary = 0.9f;
-        const float marginal = (1 - primary) / (N - 1);
-        return sum * marginal + picked * (primary - marginal);
-    }
+    // Single components are picked among values read beforehand, the indices written out.  In a loop the
+    // compiler puts sel in place of the counter that equals it, and loads in the arms of a conditional
+    // become one load from a chosen address: either way the spectrum, and the BSDF around it, would
+    // stay in scratch memory.
     __device__ __forceinline__ float get(uint32_t sel) const {
-        float r = v[0];
-#pragma unroll
-        for (int i = 1; i < N; ++i) if (i == static_cast<int>(sel)) r = v[i];
-        return r;
+        const float a = v[0], b = v[1], c = v[2], d = v[N - 1];
+        float r = sel == 1 ? b : a;
+        r = sel == 2 ? c : r;
+        return N > 3 && sel == 3 ? d : r;
     }
     __device__ __forceinline__ void set(uint32_t sel, float x) {
+        const float a = v[0], b = v[1], c = v[2], d = v[N - 1];
+        v[0] = sel == 0 ? x : a;
+        v[1] = sel == 1 ? x : b;
+        v[2] = sel == 2 ? x : c;
+        if constexpr (N > 3) v[3] = sel == 3 ? x : d;
+    }
+    __device__ __forceinline__ float importance(uint32_t sel) const {
+        float sum = 0;
 #pragma unroll
-        for (int i = 0; i < N; ++i) if (i == static_cast<int>(sel)) v[i] = x;
+        for (int i = 0; i < N; ++i) sum += v[i];
+        const float primary = 0.9f;
+        const float marginal = (1 - primary) / (N - 1);
+        return sum * marginal + get(sel) * (primary - marginal);
     }
 };
 template <int N> __device__ __forceinline__ Spec<N> operator*(float s, const Spec<N> &c) { return c * s; }
+// (a reference chosen at run time would keep both spectra in scratch memory)
+template <int N> __device__ __forceinline__ Spec<N> selectSpec(bool first, const Spec<N> &a, const Spec<N> &b) {
+    Spec<N> r;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const float x = a.v[i], y = b.v[i];
+        r.v[i] = first ? x : y;
+    }
+    return r;
+}
 template <int N> __device__ __forceinline__ Spec<N> lerpSpec(const Spec<N> &a, const Spec<N> &b, float t) {
     return a * (1 - t) + b * t;
 }
@@ -106,9 +119,33 @@ struct Wls {
     __device__ __forceinline__ float lambda(int i) const { return 360.0f + (830.0f - 360.0f) * (i + offset) / N; }
 };
 
+// The bins of the Meng tables that a set of wavelengths reads: bin[i] and bin[i] + 1, blended by
+// t[i].  A vertex evaluates up to five spectra at its wavelengths; the bins cost as much as one of
+// them, so they are computed once.
+template <int N>
+struct SpecBins {
+    __device__ __forceinline__ explicit SpecBins(const Wls<N> &) {}
+};
+template <>
+struct SpecBins<4> {
+    uint32_t bin[4];
+    float t[4];
+    __device__ __forceinline__ explicit SpecBins(const Wls<4> &wls) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float p = (wls.lambda(i) - 360.0f) / (830.0f - 360.0f);
+            p = fminf(fmaxf(p, 0.0f), 1.0f);
+            const float f = p * (95 - 1);
+            // the last sample is the upper end of the last pair of bins (t = 1)
+            bin[i] = min(static_cast<uint32_t>(f), 93u);
+            t[i] = f - bin[i];
+        }
+    }
+};
+
 // Meng et al. 2015 evaluation (spectrum_types.cpp:273-336)
 __device__ __forceinline__ Spec<4> mengEvaluate(const DevScene &sc, uint32_t adj, uint32_t st, float scale,
-                                                const Wls<4> &wls) {
+                                                const SpecBins<4> &bins) {
     uint32_t a0 = adj & 0xFF, a1 = (adj >> 8) & 0xFF, a2 = (adj >> 16) & 0xFF, a3 = (adj >> 24) & 0xFF;
     float sf = static_cast<float>(st & 0xFFFF) / (65535 - 1);
     float tf = static_cast<float>(st >> 16) / (65535 - 1);
@@ -125,26 +162,25 @@ __device__ __forceinline__ Spec<4> mengEvaluate(const DevScene &sc, uint32_t adj
         w2 = 1.0f - sf - tf;
         w3 = 0.0f;
     }
+    // a pair of neighbouring samples is one 8-byte load
+    struct __attribute__((packed, aligned(4))) Pair { float lo, hi; };
     const float *P = sc.mengPoints;
+    auto sample = [&](uint32_t point, int i) {
+        const Pair s = *reinterpret_cast<const Pair *>(P + point * 99 + 4 + bins.bin[i]);
+        return s.lo * (1 - bins.t[i]) + s.hi * bins.t[i];
+    };
     Spec<4> ret(0.0f);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        float p = (wls.lambda(i) - 360.0f) / (830.0f - 360.0f);
-        p = fminf(fmaxf(p, 0.0f), 1.0f);
-        float sBinF = p * (95 - 1);
-        uint32_t sBin = min(static_cast<uint32_t>(sBinF), 94u);
-        uint32_t sNext = min(sBin + 1, 94u);
-        float t = sBinF - sBin;
-        const float *s0 = P + a0 * 99 + 4, *s1 = P + a1 * 99 + 4, *s2 = P + a2 * 99 + 4;
         float acc = 0.0f;
-        acc += w0 * (s0[sBin] * (1 - t) + s0[sNext] * t);
-        acc += w1 * (s1[sBin] * (1 - t) + s1[sNext] * t);
-        acc += w2 * (s2[sBin] * (1 - t) + s2[sNext] * t);
-        if (quad) {
-            const float *s3 = P + a3 * 99 + 4;
-            acc += w3 * (s3[sBin] * (1 - t) + s3[sNext] * t);
-        }
+        acc += w0 * sample(a0, i);
+        acc += w1 * sample(a1, i);
+        acc += w2 * sample(a2, i);
         ret[i] = acc;
+    }
+    if (quad) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ret[i] += w3 * sample(a3, i);
     }
     return ret * scale;
 }
@@ -155,25 +191,28 @@ __device__ __forceinline__ void mengAdjacents(const DevScene &sc, float u, float
     v = fminf(fmaxf(v, 0.0f), 14.0f);
     // u == 12 or v == 14 would index one cell past the grid; stay on the last cell
     int32_t ui = min(static_cast<int32_t>(u), 11), vi = min(static_cast<int32_t>(v), 13);
-    const MengCellDev cell = sc.mengGrid[ui + 12 * vi];
+    // the cell's eight bytes as one word: a run-time index into a copy would keep it in scratch memory
+    const uint64_t cell = *reinterpret_cast<const uint64_t *>(sc.mengGrid + ui + 12 * vi);
+    const auto point = [&](int k) { return static_cast<uint32_t>(cell >> (16 + 8 * k)) & 0xFFu; };
+    const int numPoints = static_cast<int>(cell >> 8) & 0xFF;
     uint32_t adj = 0, st = 0;
-    if (cell.inside) {
+    if (cell & 0xFFu) {
         float s = u - ui, t = v - vi;
-        adj = (uint32_t(cell.idx[3]) << 24) | (uint32_t(cell.idx[2]) << 16) | (uint32_t(cell.idx[1]) << 8) | cell.idx[0];
+        adj = (point(3) << 24) | (point(2) << 16) | (point(1) << 8) | point(0);
         uint32_t ss = static_cast<uint16_t>(fmaxf(s * (65535 - 1), 0.0f));
         uint32_t tt = static_cast<uint16_t>(fmaxf(t * (65535 - 1), 0.0f));
         st = ss | (tt << 16);
-    } else if (cell.numPoints >= 3) {
+    } else if (numPoints >= 3) {
         // cells with no data points lie outside the spectral locus; their (u, v) keeps adj = 0
         const float *P = sc.mengPoints;
-        const uint32_t i0 = cell.idx[0];
+        const uint32_t i0 = point(0);
         const float ex = u - P[i0 * 99 + 2];
         const float ey = v - P[i0 * 99 + 3];
-        float e0x = P[cell.idx[1] * 99 + 2] - P[i0 * 99 + 2];
-        float e0y = P[cell.idx[1] * 99 + 3] - P[i0 * 99 + 3];
+        float e0x = P[point(1) * 99 + 2] - P[i0 * 99 + 2];
+        float e0y = P[point(1) * 99 + 3] - P[i0 * 99 + 3];
         float uu = e0x * ey - ex * e0y;
-        for (int i = 1; i < cell.numPoints; ++i) {
-            uint32_t idx = cell.idx[i % (cell.numPoints - 1) + 1];
+        for (int i = 1; i < numPoints; ++i) {
+            uint32_t idx = point(i % (numPoints - 1) + 1);
             float e1x = P[idx * 99 + 2] - P[i0 * 99 + 2];
             float e1y = P[idx * 99 + 3] - P[i0 * 99 + 3];
             float vv = ex * e1y - e1x * ey;
@@ -187,7 +226,7 @@ __device__ __forceinline__ void mengAdjacents(const DevScene &sc, float u, float
                 e0y = e1y;
                 continue;
             }
-            adj = (0xFFu << 24) | (i0 << 16) | (uint32_t(cell.idx[i]) << 8) | idx;
+            adj = (0xFFu << 24) | (i0 << 16) | (point(i) << 8) | idx;
             uint32_t ss = static_cast<uint16_t>(fmaxf(b0 * (65535 - 1), 0.0f));
             uint32_t tt = static_cast<uint16_t>(fmaxf(b1 * (65535 - 1), 0.0f));
             st = ss | (tt << 16);
@@ -199,14 +238,18 @@ __device__ __forceinline__ void mengAdjacents(const DevScene &sc, float u, float
 }
 
 template <int N>
-__device__ __forceinline__ Spec<N> evalSpectrum(const DevScene &sc, const DevSpectrum &p, const Wls<N> &wls) {
+__device__ __forceinline__ Spec<N> evalSpectrum(const DevScene &sc, const DevSpectrum &p, const SpecBins<N> &bins) {
     if constexpr (N == 3) {
         Spec<3> r;
         r[0] = p.x; r[1] = p.y; r[2] = p.z;
         return r;
     } else {
-        return mengEvaluate(sc, __float_as_uint(p.x), __float_as_uint(p.y), p.z, wls);
+        return mengEvaluate(sc, __float_as_uint(p.x), __float_as_uint(p.y), p.z, bins);
     }
+}
+template <int N>
+__device__ __forceinline__ Spec<N> evalSpectrum(const DevScene &sc, const DevSpectrum &p, const Wls<N> &wls) {
+    return evalSpectrum<N>(sc, p, SpecBins<N>(wls));
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -232,12 +275,16 @@ __device__ __forceinline__ void concentricSampleDisk(float u0, float u1, float *
         *dy = 0;
         return;
     }
-    if (sx >= -sy) {
-        if (sx > sy) { r = sx; theta = sy / sx; }
-        else { r = sy; theta = 2 - sx / sy; }
+    // the quarter of the square picks the larger coordinate's sign and the angle's offset; the four
+    // share one division
+    const bool right = sx >= -sy, wide = right == (sx > sy);
+    const float q = wide ? sy / sx : sx / sy;
+    r = wide ? sx : sy;
+    if (right) {
+        theta = wide ? q : 2 - q;
     } else {
-        if (sx > sy) { r = -sy; theta = 6 + sx / sy; }
-        else { r = -sx; theta = 4 + sy / sx; }
+        r = -r;
+        theta = wide ? 4 + q : 6 + q;
     }
     theta *= kPiF / 4;
     float s, c;
@@ -340,14 +387,15 @@ struct Ggx {
         float a2t2 = (sq(vr.x * ax) + sq(vr.y * ay)) / sq(vr.z);
         return (-1 + sqrtf(1 + a2t2)) / 2;
     }
+    // 1 where dot(v, m) / v.z > 0: the two have the same sign
+    static __device__ __forceinline__ float facing(float dotVM, float vz) {
+        return __uint_as_float(__float_as_uint(dotVM) ^ (__float_as_uint(vz) & 0x80000000u)) > 0 ? 1.0f : 0.0f;
+    }
     __device__ __forceinline__ float G1(const V3 &v, const V3 &m) const {
-        float chi = (dot(v, m) / v.z) > 0 ? 1.0f : 0.0f;
-        return chi / (1 + lambda(v));
+        return facing(dot(v, m), v.z) / (1 + lambda(v));
     }
     __device__ __forceinline__ float Gcorr(const V3 &v1, const V3 &v2, const V3 &m) const {
-        float chi1 = (dot(v1, m) / v1.z) > 0 ? 1.0f : 0.0f;
-        float chi2 = (dot(v2, m) / v2.z) > 0 ? 1.0f : 0.0f;
-        return chi1 * chi2 / (1 + lambda(v1) + lambda(v2));
+        return facing(dot(v1, m), v1.z) * facing(dot(v2, m), v2.z) / (1 + lambda(v1) + lambda(v2));
     }
     // visible-normal sampling (materials.cu:184-223)
     __device__ __forceinline__ float sample(const V3 &v, float u0, float u1, V3 *m, float *normalPDF) const {
@@ -367,8 +415,7 @@ struct Ggx {
         V3 mr = P1 * T1 + P2 * T2 + sqrtf(1.0f - P1 * P1 - P2 * P2) * sv;
         mr = normalize(V3(ax * mr.x, ay * mr.y, mr.z));
         float d = D(mr);
-        float chi = (dot(vr, mr) / vr.z) > 0 ? 1.0f : 0.0f;
-        *normalPDF = chi / (1 + lambda(vr)) * absDot(vr, mr) * d / fabsf(vr.z);
+        *normalPDF = facing(dot(vr, mr), vr.z) / (1 + lambda(vr)) * absDot(vr, mr) * d / fabsf(vr.z);
         *m = V3(cr * mr.x - sr * mr.y, sr * mr.x + cr * mr.y, mr.z);
         return d;
     }
@@ -486,8 +533,8 @@ struct Bsdf {
         }
         case BSDF_SPEC_BSDF: {
             bool entering = q.z >= 0.0f;
-            const Spec<N> &eEnter = entering ? c1 : c2;
-            const Spec<N> &eExit = entering ? c2 : c1;
+            const Spec<N> eEnter = selectSpec<N>(entering, c1, c2);
+            const Spec<N> eExit = selectSpec<N>(entering, c2, c1);
             V3 v = entering ? q : -q;
             Spec<N> F = fresnelDielectric<N>(eEnter, eExit, v.z);
             float reflectProb = F.importance(wl);
@@ -600,8 +647,8 @@ struct Bsdf {
         case BSDF_MICRO_BSDF: {
             // materials.cu:1270-1368
             bool entering = q.z >= 0.0f;
-            const Spec<N> &eEnter = entering ? c1 : c2;
-            const Spec<N> &eExit = entering ? c2 : c1;
+            const Spec<N> eEnter = selectSpec<N>(entering, c1, c2);
+            const Spec<N> eExit = selectSpec<N>(entering, c2, c1);
             Ggx g(a0, a1, a2);
             V3 v = entering ? q : -q;
             V3 m;
@@ -677,7 +724,7 @@ struct Bsdf {
         }
     }
 
-    __device__ Spec<N> evaluateInternal(const V3 &q, const V3 &d, uint32_t wl, bool importance,
+    __device__ __forceinline__ Spec<N> evaluateInternal(const V3 &q, const V3 &d, uint32_t wl, bool importance,
                                         Spec<N> *revValue) const {
         Spec<N> ret(0.0f);
         switch (kind) {
@@ -715,8 +762,8 @@ struct Bsdf {
         }
         case BSDF_MICRO_BSDF: {
             bool entering = q.z >= 0.0f;
-            const Spec<N> &eEnter = entering ? c1 : c2;
-            const Spec<N> &eExit = entering ? c2 : c1;
+            const Spec<N> eEnter = selectSpec<N>(entering, c1, c2);
+            const Spec<N> eExit = selectSpec<N>(entering, c2, c1);
             Ggx g(a0, a1, a2);
             V3 v = entering ? q : -q;
             V3 l = entering ? d : -d;
@@ -750,7 +797,7 @@ struct Bsdf {
         return ret;
     }
 
-    __device__ float evaluatePDFInternal(const V3 &q, const V3 &d, uint32_t wl, float *revPDF) const {
+    __device__ __forceinline__ float evaluatePDFInternal(const V3 &q, const V3 &d, uint32_t wl, float *revPDF) const {
         if (revPDF) *revPDF = 0.0f;
         switch (kind) {
         case BSDF_MATTE:
@@ -788,8 +835,8 @@ struct Bsdf {
             // materials.cu:1462-1510; the transmission half vector carries no sign flip for
             // queries from inside, as in the reference
             bool entering = q.z >= 0.0f;
-            const Spec<N> &eEnter = entering ? c1 : c2;
-            const Spec<N> &eExit = entering ? c2 : c1;
+            const Spec<N> eEnter = selectSpec<N>(entering, c1, c2);
+            const Spec<N> eExit = selectSpec<N>(entering, c2, c1);
             V3 v = entering ? q : -q;
             V3 l = entering ? d : -d;
             float nn = l.z * v.z;
@@ -851,6 +898,30 @@ struct Bsdf {
         if (revPDF) *revPDF = 0.0f;
         if (!matches(dt::All)) return 0.0f;
         return evaluatePDFInternal(q, d, wl, revPDF);
+    }
+    // evaluate and evaluatePDF of one direction for radiance transport: per kind the two share
+    // their half vector, distribution and masking terms
+    __device__ __forceinline__ Spec<N> evaluateWithPDF(const V3 &q, const V3 &gnL, const V3 &d, uint32_t wl,
+                                                       float *pdf) const {
+        Spec<N> f(0.0f);
+        *pdf = 0.0f;
+        switch (kind) {
+        case BSDF_MATTE: f = valueAndPDF<BSDF_MATTE>(q, d, wl, pdf); break;
+        case BSDF_MICRO_BRDF: f = valueAndPDF<BSDF_MICRO_BRDF>(q, d, wl, pdf); break;
+        case BSDF_DIFFSPEC: f = valueAndPDF<BSDF_DIFFSPEC>(q, d, wl, pdf); break;
+        case BSDF_MICRO_BSDF: f = valueAndPDF<BSDF_MICRO_BSDF>(q, d, wl, pdf); break;
+        default: break;   // deltas evaluate to zero
+        }
+        const float sn = fabsf(d.z / dot(d, gnL));
+        return isfinite(sn) ? f * sn : Spec<N>(0.0f);
+    }
+    template <uint32_t KIND>
+    __device__ __forceinline__ Spec<N> valueAndPDF(const V3 &q, const V3 &d, uint32_t wl, float *pdf) const {
+        Bsdf b = *this;
+        b.kind = KIND;
+        const Spec<N> f = b.evaluateInternal(q, d, wl, false, nullptr);
+        *pdf = b.evaluatePDFInternal(q, d, wl, nullptr);
+        return f;
     }
 };
 

@@ -241,6 +241,10 @@ struct DevScene {
     // light selection over [environment, instances...]
     uint32_t lightInstBase;
     uint32_t numLightInsts;
+    // Entries of that distribution up to the last emitter: the CDF is 1 past it, so no number below
+    // 1 falls further, and the search skips the instances that emit nothing (all of them where only
+    // the environment does).
+    uint32_t numLightInstsSearched;
     float lightInstIntegral;
     // environment
     uint32_t hasEnv;

@@ -73,22 +73,24 @@ constexpr int kTraceLds = 2 * kLdsStack * kTraceBlock;
 // A CU's 160 KB of LDS holds 9 blocks of kTraceLds (4.5 waves per SIMD).  The per-depth
 // closest-hit kernel keeps 12 entries per lane (12 KB per block), so that its registers (5 waves
 // per SIMD) set the limit; the per-depth any-hit kernel needs no entry distances (8 KB per block
-// for 16 entries; 7 waves per SIMD).  The tail kernel, limited to 4 waves per SIMD by its
+// for 16 entries; 7 waves per SIMD).  The tail kernel, limited to 3 waves per SIMD by its
 // registers, keeps the full kTraceLds.
 constexpr int kIntersectStack = 12;
 constexpr int kIntersectLds = 2 * kIntersectStack * kTraceBlock;
 constexpr int kShadowLds = kLdsStack * kTraceBlock;
-#ifndef VLRA_TAIL_WAVES_PER_EU
-#define VLRA_TAIL_WAVES_PER_EU 4
-#endif
-constexpr int kTailWavesPerEU = VLRA_TAIL_WAVES_PER_EU;   // occupancy asked of the tail kernel
+// Occupancy asked of the tail kernel.  It holds a path, a ray and a shading vertex; at 4 waves per SIMD
+// (128 VGPRs) it spilled 60 to 130 of them into its loops.  Measured at 4 / 3 waves: textured 720p
+// 3.95 / 3.49 ms (4 frames), cached 1080p 10.1 / 9.3 ms (8), Cornell box 256 x 256 4.78 / 4.63 ms (16),
+// icosphere grid 1080p 22.5 / 22.9 ms (8); at 2 waves the grid takes 26.3 ms.
+constexpr int kTailWavesPerEU = 3;
 // Occupancy asked of the per-path LVC-BPT and light-tracing kernels.  Left to themselves they
 // take 130-230 VGPRs and run 2 waves per SIMD; with some registers spilled, more waves hide
 // more of their traversals' fetch latency (C3 box at 1280x720: light paths 1.55 -> 1.39 ms,
-// eye paths 2.40 -> 1.89 ms, light tracing 2.60 -> 1.79 ms per frame).
+// eye paths 2.40 -> 1.89 ms per frame).  Light tracing: 3 waves 3.61 ms, 4 waves 3.80 ms for 4 frames
+// at 720p; LVC-BPT with one wave fewer for both kernels 7.85 ms in place of 6.93 ms.
 constexpr int kBptLightWavesPerEU = 4;
 constexpr int kBptEyeWavesPerEU = 3;
-constexpr int kLightTraceWavesPerEU = 4;
+constexpr int kLightTraceWavesPerEU = 3;
 constexpr int32_t kSentinel = INT32_MIN;
 
 // ---------------------------------------------------------------------------------------------
@@ -480,19 +482,29 @@ __device__ __forceinline__ uint32_t appendSlot(uint32_t *counter, bool active) {
 // distributions (shared.h:182-298)
 __device__ __forceinline__ uint32_t nextPow2(uint32_t x) { return x <= 1 ? 1 : 1u << (32 - __clz(x - 1)); }
 
+// The last of the n ascending entries that is <= u (entry 0 counts as such), by steps of falling
+// powers of two.  Each round takes two of them at once: its three entries are loaded together, so a
+// search waits for half as many dependent loads.
 __device__ __forceinline__ uint32_t discreteSearch(const float *cdf, uint32_t n, float u) {
-    int idx = 0;
-    for (int d = static_cast<int>(nextPow2(n) >> 1); d >= 1; d >>= 1) {
-        if (idx + d >= static_cast<int>(n)) continue;
-        if (cdf[idx + d] <= u) idx += d;
+    uint32_t idx = 0, d = nextPow2(n) >> 1;
+    if (__clz(d) & 1) {   // an odd number of steps: d = 1, 4, 16, ...
+        if (d < n && cdf[d] <= u) idx = d;
+        d >>= 1;
     }
-    return static_cast<uint32_t>(idx);
+    for (d >>= 1; d; d >>= 2) {
+        const uint32_t i1 = idx + d, i2 = i1 + d, i3 = i2 + d;
+        const float c1 = cdf[min(i1, n)], c2 = cdf[min(i2, n)], c3 = cdf[min(i3, n)];
+        const bool in1 = i1 < n && c1 <= u, in2 = i2 < n && c2 <= u, in3 = i3 < n && c3 <= u;
+        idx = in2 ? (in3 ? i3 : i2) : (in1 ? i1 : idx);
+    }
+    return idx;
 }
 // Discrete1D: PMF at base, CDF (n + 1 entries) after it
-__device__ __forceinline__ uint32_t sampleDiscrete(const float *pool, uint32_t base, uint32_t n, float u, float *prob,
-                                                   float *remapped) {
+// (searched: the entries that u can fall on, when fewer than n)
+__device__ __forceinline__ uint32_t sampleDiscrete(const float *pool, uint32_t base, uint32_t n, uint32_t searched,
+                                                   float u, float *prob, float *remapped) {
     const float *pmf = pool + base, *cdf = pool + base + n;
-    uint32_t idx = discreteSearch(cdf, n, u);
+    uint32_t idx = discreteSearch(cdf, searched, u);
     *prob = pmf[idx];
     if (remapped) *remapped = (u - cdf[idx]) / (cdf[idx + 1] - cdf[idx]);
     return idx;
@@ -522,15 +534,16 @@ __device__ __forceinline__ float envMapPDF(const DevScene &sc, float d0, float d
            continuousPDF(sc.distPool, sc.envRowBase + row * (2 * sc.envMapW + 1), sc.envMapW, d0);
 }
 
-// bilinear environment fetch, repeat wrapping in both axes
+// bilinear environment fetch, repeat wrapping in both axes (u and v lie in [0, 1], so the texels
+// left of and right of the sample are at most one past the edges)
 __device__ __forceinline__ float4 envFetch(const DevScene &sc, float u, float v) {
     float x = u * sc.envW - 0.5f, y = v * sc.envH - 0.5f;
     float fx0 = floorf(x), fy0 = floorf(y);
     float wx = x - fx0, wy = y - fy0;
-    int32_t x0 = static_cast<int32_t>(fx0), y0 = static_cast<int32_t>(fy0);
-    int32_t W = static_cast<int32_t>(sc.envW), H = static_cast<int32_t>(sc.envH);
-    int32_t xa = ((x0 % W) + W) % W, xb = (((x0 + 1) % W) + W) % W;
-    int32_t ya = ((y0 % H) + H) % H, yb = (((y0 + 1) % H) + H) % H;
+    const int32_t W = static_cast<int32_t>(sc.envW), H = static_cast<int32_t>(sc.envH);
+    const int32_t x0 = min(max(static_cast<int32_t>(fx0), -1), W - 1), y0 = min(max(static_cast<int32_t>(fy0), -1), H - 1);
+    const int32_t xa = x0 < 0 ? W - 1 : x0, xb = x0 + 1 < W ? x0 + 1 : 0;
+    const int32_t ya = y0 < 0 ? H - 1 : y0, yb = y0 + 1 < H ? y0 + 1 : 0;
     float4 t00 = sc.envTex[ya * W + xa], t10 = sc.envTex[ya * W + xb];
     float4 t01 = sc.envTex[yb * W + xa], t11 = sc.envTex[yb * W + xb];
     float4 r;
@@ -543,10 +556,10 @@ __device__ __forceinline__ float4 envFetch(const DevScene &sc, float u, float v)
 
 template <int N>
 __device__ __forceinline__ Spec<N> envEmittance(const DevScene &sc, const DevMaterial &m, float texU, float texV,
-                                                const Wls<N> &wls) {
+                                                const SpecBins<N> &bins) {
     Spec<N> e;
     if (!m.useEnvTexture || sc.envTex == nullptr) {
-        e = evalSpectrum<N>(sc, m.spec[0], wls);
+        e = evalSpectrum<N>(sc, m.spec[0], bins);
     } else {
         float4 t = envFetch(sc, texU, texV);
         if constexpr (N == 3) {
@@ -554,7 +567,7 @@ __device__ __forceinline__ Spec<N> envEmittance(const DevScene &sc, const DevMat
         } else {
             uint32_t adj, st;
             mengAdjacents(sc, t.x, t.y, &adj, &st);
-            e = mengEvaluate(sc, adj, st, t.z / 0.009355121400914532f, wls);
+            e = mengEvaluate(sc, adj, st, t.z / 0.009355121400914532f, bins);
         }
     }
     return e * m.scalars[0];
@@ -617,7 +630,9 @@ __device__ __forceinline__ float alphaAt(const DevScene &sc, int32_t inst, uint3
 // environment surface point from a direction (path_tracing.cu:282-310)
 __device__ __forceinline__ void envPointFromDir(const DevScene &sc, const V3 &direction, SurfPt *sp, float *hypAreaPDF) {
     float theta = acosf(fminf(fmaxf(direction.y, -1.0f), 1.0f));
-    float phi = fmodf(atan2f(-direction.x, direction.z) + 2 * kPiF, 2 * kPiF);
+    // fmod(atan2 + 2 pi, 2 pi): the sum lies in [pi, 3 pi], where one subtraction (exact) does it
+    float phi = atan2f(-direction.x, direction.z) + 2 * kPiF;
+    if (phi >= 2 * kPiF) phi -= 2 * kPiF;
     float sinPhi, cosPhi;
     sincosf(phi, &sinPhi, &cosPhi);
     V3 tc0 = normalize(V3(-cosPhi, 0.0f, -sinPhi));
@@ -651,7 +666,8 @@ struct LightSample {
 __device__ __forceinline__ void sampleLight(const DevScene &sc, float uLight, float uP0, float uP1, LightSample *ls,
                                             float *lightProb) {
     float instProb, uInst;
-    uint32_t li = sampleDiscrete(sc.distPool, sc.lightInstBase, sc.numLightInsts, uLight, &instProb, &uInst);
+    uint32_t li = sampleDiscrete(sc.distPool, sc.lightInstBase, sc.numLightInsts, sc.numLightInstsSearched, uLight,
+                                 &instProb, &uInst);
     if (li == 0) {
         *lightProb = instProb;
         float u, v, uvPDF;
@@ -660,9 +676,10 @@ __device__ __forceinline__ void sampleLight(const DevScene &sc, float uLight, fl
         float theta = kPiF * v;
         float posPhi = phi - sc.envRotation;
         posPhi = posPhi - floorf(posPhi / (2 * kPiF)) * 2 * kPiF;
-        V3 dir = fromPolarYUp(posPhi, theta);
-        float sinPhi, cosPhi;
+        float sinPhi, cosPhi, sinTheta, cosTheta;
         sincosf(posPhi, &sinPhi, &cosPhi);
+        sincosf(theta, &sinTheta, &cosTheta);
+        const V3 dir(-sinPhi * sinTheta, cosTheta, cosPhi * sinTheta);
         V3 tc0 = normalize(V3(-cosPhi, 0.0f, -sinPhi));
         V3 gn = -dir;
         ls->sp.position = dir;
@@ -677,19 +694,19 @@ __device__ __forceinline__ void sampleLight(const DevScene &sc, float uLight, fl
         ls->sp.instIndex = ls->sp.geomInstIndex = ls->sp.primIndex = 0;
         ls->sp.u = posPhi;
         ls->sp.v = theta;
-        ls->areaPDF = uvPDF / (2 * kPiF * kPiF * sinf(theta));
+        ls->areaPDF = uvPDF / (2 * kPiF * kPiF * sinTheta);
         ls->posType = dt::Reflection | dt::LowFreq;
         ls->material = sc.envMaterial;
         return;
     }
     const DevInstance &I = sc.instances[li - 1];
     float geomProb, uPrim;
-    uint32_t lgi = sampleDiscrete(sc.distPool, I.lightDistBase, I.numGeomInsts, uInst, &geomProb, &uPrim);
+    uint32_t lgi = sampleDiscrete(sc.distPool, I.lightDistBase, I.numGeomInsts, I.numGeomInsts, uInst, &geomProb, &uPrim);
     uint32_t gi = sc.instGeomInsts[I.geomInstListBase + lgi];
     const DevGeomInst &G = sc.geomInsts[gi];
     *lightProb = instProb * geomProb;
     float primProb;
-    uint32_t prim = sampleDiscrete(sc.distPool, G.distBase, G.numPrims, uPrim, &primProb, nullptr);
+    uint32_t prim = sampleDiscrete(sc.distPool, G.distBase, G.numPrims, G.numPrims, uPrim, &primProb, nullptr);
     ls->material = G.material;
     ls->sp.instIndex = li - 1;
     ls->sp.geomInstIndex = gi;
@@ -746,13 +763,13 @@ __device__ __forceinline__ void sampleLight(const DevScene &sc, float uLight, fl
 // returns emittance M (evaluateEmittance) and the directional factor for dirLocal.
 template <int N, bool NODES = true>
 __device__ __forceinline__ bool evalEDF(const DevScene &sc, const DevMaterial &m, const SurfPt &sp, const Wls<N> &wls,
-                                        const V3 &dirLocal, Spec<N> *M, float *fe) {
+                                        const SpecBins<N> &bins, const V3 &dirLocal, Spec<N> *M, float *fe) {
     switch (m.type) {
     case MAT_DIFFUSE_EMITTER: {
         NodeOutputs<N> o;
         if constexpr (NODES) materialNodes<N>(sc, m, &sp, wls, &o);
         else o.has = 0;
-        *M = materialSpectrum<N>(sc, m, 0, o, wls) * m.scalars[0];
+        *M = materialSpectrum<N>(sc, m, 0, o, bins) * m.scalars[0];
         *fe = dirLocal.z > 0.0f ? 1.0f / kPiF : 0.0f;
         return true;
     }
@@ -760,17 +777,23 @@ __device__ __forceinline__ bool evalEDF(const DevScene &sc, const DevMaterial &m
         NodeOutputs<N> o;
         if constexpr (NODES) materialNodes<N>(sc, m, &sp, wls, &o);
         else o.has = 0;
-        *M = materialSpectrum<N>(sc, m, 0, o, wls) * m.scalars[0];
+        *M = materialSpectrum<N>(sc, m, 0, o, bins) * m.scalars[0];
         *fe = 1.0f / (4 * kPiF);
         return true;
     }
     case MAT_ENVIRONMENT_EMITTER:
-        *M = kPiF * envEmittance<N>(sc, m, sp.texU, sp.texV, wls);
+        *M = kPiF * envEmittance<N>(sc, m, sp.texU, sp.texV, bins);
         *fe = dirLocal.z > 0.0f ? 1.0f / kPiF : 0.0f;
         return true;
     default:
         return false;
     }
+}
+
+template <int N, bool NODES = true>
+__device__ __forceinline__ bool evalEDF(const DevScene &sc, const DevMaterial &m, const SurfPt &sp, const Wls<N> &wls,
+                                        const V3 &dirLocal, Spec<N> *M, float *fe) {
+    return evalEDF<N, NODES>(sc, m, sp, wls, SpecBins<N>(wls), dirLocal, M, fe);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1143,6 +1166,9 @@ __device__ __forceinline__ void writeCacheRecord(const DevScene &sc, const SurfP
 // One bounce of path_tracing.cu:133-337 for a ray that hit (ha.x >= 0) or missed: implicit
 // emission with MIS, Russian roulette, next-event estimation (returns the shadow ray and the
 // contribution it carries when unoccluded) and BSDF sampling (returns the next ray).
+// A wave's lanes miss, hit emitters and hit surfaces at once, and each kind needs some emitter's
+// emittance (the environment's, its own, the sampled light's): it is evaluated in one place for all
+// of them, as are the spectra of the materials (setupBsdf), in place of once per kind.
 template <int N, bool NODES = true>
 __device__ __forceinline__ void shadeStep(const DevScene &sc, uint32_t pathLength, uint32_t maxPathLength,
                                           uint32_t path, const V3 &rayOrg, const V3 &rayDir, int4 ha, float2 hb,
@@ -1162,163 +1188,183 @@ __device__ __forceinline__ void shadeStep(const DevScene &sc, uint32_t pathLengt
             cc.b.trainAfterStamp[slot] = cc.stamp;
         }
     }
-    if (ha.x < 0) {
-        // miss: environment light with MIS
+    const SpecBins<N> bins(P.wls);
+    const bool miss = ha.x < 0;
+    SurfPt sp;
+    Bsdf<N> bsdf;
+    V3 dirOutLocal, gnL;
+    float hypAreaPDF = 0.0f;
+    bool cacheEnd = false;
+    bool goesOn = false;          // the path has survived this vertex's Russian roulette
+    uint32_t trainSlot = ~0u;     // the training sample whose contribution is recorded after the emission
+    const Spec<N> alphaIn = P.alpha;
+    // the emitter point: where an escaped ray meets the environment, the hit point on an emitter, or
+    // the light sample of the next-event estimate (an emitter's surface makes none)
+    LightSample ls;
+    float lightProb = 0.0f;
+    V3 sdir, emitDir;
+    float dist2 = 0.0f;
+    bool emission = false, nextEvent = false;
+    if (miss) {
+        // environment light with MIS
         if (sc.hasEnv && sc.envImportance > 0.0f) {
-            SurfPt sp;
-            float hypAreaPDF;
-            envPointFromDir(sc, rayDir, &sp, &hypAreaPDF);
-            const DevMaterial &m = sc.materials[sc.envMaterial];
-            V3 dirOutLocal = sp.frame.toLocal(-rayDir);
-            Spec<N> M;
-            float fe;
-            evalEDF<N, NODES>(sc, m, sp, P.wls, dirOutLocal, &M, &fe);
-            if (!M.isZero()) {
-                float mis = 1.0f;
-                if (!dt::isDelta(P.prevType) && pathLength > 1) {
-                    float instProb = 1.0f / sc.lightInstIntegral;
-                    float bsdfPDF = P.prevDirPDF;
-                    float lightPDF = instProb * hypAreaPDF * 1.0f / fabsf(dirOutLocal.z);
-                    mis = (bsdfPDF * bsdfPDF) / (lightPDF * lightPDF + bsdfPDF * bsdfPDF);
+            envPointFromDir(sc, rayDir, &ls.sp, &hypAreaPDF);
+            ls.material = sc.envMaterial;
+            dirOutLocal = ls.sp.frame.toLocal(-rayDir);
+            emitDir = dirOutLocal;
+            emission = true;
+        }
+    } else {
+        decodeHit<NODES>(sc, ha.x, ha.y, ha.z, hb.x, hb.y, &sp, &hypAreaPDF);
+        const DevGeomInst &G = sc.geomInsts[ha.y];
+        const DevMaterial &mat = sc.materials[G.material];
+        dirOutLocal = sp.frame.toLocal(-rayDir);
+        if (mat.isEmitter) {
+            if constexpr (NODES) {
+                ls.sp = sp;
+            } else {
+                ls.sp.texU = sp.texU;
+                ls.sp.texV = sp.texV;
+            }
+            ls.material = G.material;
+            emitDir = dirOutLocal;
+            emission = true;
+        }
+        if (cc.mode != 0) {
+            // path spread (Mueller et al. 2021, "Real-time Neural Radiance Caching for Path
+            // Tracing"): a_0 from the primary vertex, then one term per non-delta bounce
+            const float d2 = (sp.position - rayOrg).sqLength();
+            const float cosT = fabsf(dirOutLocal.z);
+            if (pathLength == 1) {
+                P.a0 = sqrtf(d2 / (4 * kPiF * cosT));
+                P.a = 0.0f;
+            } else if (!dt::isDelta(P.prevType)) {
+                P.a += sqrtf(d2 / (P.prevDirPDF * cosT));
+            }
+            const uint32_t pix = (path / cc.width) * cc.imageW + path % cc.width;
+            if (pix % cc.stride == cc.offset) {
+                // training path: vertices 1..kCacheTrainVerts become samples once the path ends
+                if (pathLength <= kCacheTrainVerts) {
+                    const uint32_t slot = (pix / cc.stride) * kCacheTrainVerts + pathLength - 1;
+                    writeCacheRecord(sc, sp, G.material, rayDir, N == 4 ? P.wls.offset : 0.0f, cc.b.trainRaw + 4 * slot);
+                    cc.b.trainThroughput[slot] = storeSpec<N>(P.alpha);
+                    cc.b.trainStamp[slot] = cc.stamp;
+                    // the sample is everything the path gathers after this vertex's emission
+                    if (cc.full) trainSlot = slot;
                 }
-                P.contrib += P.alpha * (M * fe) * mis;
+            } else {
+                cacheEnd = cc.mode == 2 && pathLength >= 2 && !maxLengthTerminate && !P.wls.single &&
+                           P.a > cc.threshold * P.a0;
             }
         }
-        return;
+        auto roulette = [&]() {
+            const float continueProb = fminf(P.alpha.importance(P.wls.sel) / P.initImportance, 1.0f);
+            const bool survives = !(P.rng.uniform() >= continueProb);
+            if (survives) P.alpha = P.alpha / continueProb;
+            return survives;
+        };
+        if (!maxLengthTerminate) {
+            P.rngUsed = true;
+            goesOn = cacheEnd || roulette();
+        }
+        if (goesOn) {
+            bsdf = setupBsdf<N, NODES>(sc, mat, P.wls, bins, &sp);
+            if (cacheEnd && cc.full) {
+                if (bsdf.hasNonDelta()) {
+                    // the cache supplies all the radiance this vertex reflects; no next-event estimate
+                    writeCacheRecord(sc, sp, G.material, rayDir, N == 4 ? P.wls.offset : 0.0f, cc.b.queryRaw + 4 * path);
+                    cc.b.queryThroughput[path] = storeSpec<N>(P.alpha);
+                    cc.b.queryStamp[path] = cc.stamp;
+                    goesOn = false;
+                } else {
+                    // a purely specular vertex does not end in the cache: the path goes on
+                    cacheEnd = false;
+                    goesOn = roulette();
+                }
+            }
+        }
+        if (goesOn) {
+            gnL = sp.frame.toLocal(sp.gn);
+            if (bsdf.hasNonDelta()) {
+                float uLight = P.rng.uniform();
+                float uP0 = P.rng.uniform(), uP1 = P.rng.uniform();
+                // a scene without emitters has nothing to sample (the draws are still made)
+                if (sc.lightInstIntegral > 0.0f) {
+                    sampleLight(sc, uLight, uP0, uP1, &ls, &lightProb);
+                    // shadow ray direction (SurfacePoint::calcDirectionFrom)
+                    if (ls.sp.atInfinity) {
+                        dist2 = 1.0f;
+                        sdir = normalize(ls.sp.position);
+                    } else {
+                        V3 dv = ls.sp.position - sp.position;
+                        dist2 = dv.sqLength();
+                        sdir = dv / sqrtf(dist2);
+                    }
+                    emitDir = ls.sp.frame.toLocal(-sdir);
+                    nextEvent = true;
+                }
+            }
+        }
     }
-    SurfPt sp;
-    float hypAreaPDF;
-    decodeHit<NODES>(sc, ha.x, ha.y, ha.z, hb.x, hb.y, &sp, &hypAreaPDF);
-    const DevGeomInst &G = sc.geomInsts[ha.y];
-    const DevMaterial &mat = sc.materials[G.material];
-    V3 dirOutLocal = sp.frame.toLocal(-rayDir);
-    if (mat.isEmitter) {
-        Spec<N> M;
-        float fe;
-        evalEDF<N, NODES>(sc, mat, sp, P.wls, dirOutLocal, &M, &fe);
-        if (!M.isZero()) {
-            float mis = 1.0f;
-            if (!dt::isDelta(P.prevType) && pathLength > 1) {
+    Spec<N> M(0.0f);
+    float fe = 0.0f;
+    if (emission || nextEvent)
+        evalEDF<N, NODES>(sc, sc.materials[ls.material], ls.sp, P.wls, bins, emitDir, &M, &fe);
+    if (emission && !M.isZero()) {
+        float mis = 1.0f;
+        if (!dt::isDelta(P.prevType) && pathLength > 1) {
+            float bsdfPDF = P.prevDirPDF;
+            float lightPDF;
+            if (miss) {
+                float instProb = 1.0f / sc.lightInstIntegral;
+                lightPDF = instProb * hypAreaPDF * 1.0f / fabsf(dirOutLocal.z);
+            } else {
                 const DevInstance &I = sc.instances[ha.x];
                 float instProb = I.lightDistIntegral / sc.lightInstIntegral;
-                float geomInstProb = G.importance / I.lightDistIntegral;
-                float bsdfPDF = P.prevDirPDF;
-                float dist2 = (sp.position - rayOrg).sqLength();
-                float lightPDF = instProb * geomInstProb * hypAreaPDF * dist2 / fabsf(dirOutLocal.z);
-                mis = (bsdfPDF * bsdfPDF) / (lightPDF * lightPDF + bsdfPDF * bsdfPDF);
+                float geomInstProb = sc.geomInsts[ha.y].importance / I.lightDistIntegral;
+                float d2 = (sp.position - rayOrg).sqLength();
+                lightPDF = instProb * geomInstProb * hypAreaPDF * d2 / fabsf(dirOutLocal.z);
             }
-            P.contrib += P.alpha * (M * fe) * mis;
+            mis = (bsdfPDF * bsdfPDF) / (lightPDF * lightPDF + bsdfPDF * bsdfPDF);
         }
+        P.contrib += alphaIn * (M * fe) * mis;
     }
-    bool cacheEnd = false;
-    if (cc.mode != 0) {
-        // path spread (Mueller et al. 2021, "Real-time Neural Radiance Caching for Path
-        // Tracing"): a_0 from the primary vertex, then one term per non-delta bounce
-        const float dist2 = (sp.position - rayOrg).sqLength();
-        const float cosT = fabsf(dirOutLocal.z);
-        if (pathLength == 1) {
-            P.a0 = sqrtf(dist2 / (4 * kPiF * cosT));
-            P.a = 0.0f;
-        } else if (!dt::isDelta(P.prevType)) {
-            P.a += sqrtf(dist2 / (P.prevDirPDF * cosT));
-        }
-        const uint32_t pix = (path / cc.width) * cc.imageW + path % cc.width;
-        if (pix % cc.stride == cc.offset) {
-            // training path: vertices 1..kCacheTrainVerts become samples once the path ends
-            if (pathLength <= kCacheTrainVerts) {
-                const uint32_t slot = (pix / cc.stride) * kCacheTrainVerts + pathLength - 1;
-                writeCacheRecord(sc, sp, G.material, rayDir, N == 4 ? P.wls.offset : 0.0f, cc.b.trainRaw + 4 * slot);
-                cc.b.trainThroughput[slot] = storeSpec<N>(P.alpha);
-                cc.b.trainStamp[slot] = cc.stamp;
-                if (cc.full) {
-                    // the sample is everything the path gathers after this vertex's emission
-                    cc.b.trainContrib[slot] = storeSpec<N>(P.contrib);
-                    cc.b.trainAfterStamp[slot] = cc.stamp;
-                }
-            }
-        } else {
-            cacheEnd = cc.mode == 2 && pathLength >= 2 && !maxLengthTerminate && !P.wls.single &&
-                       P.a > cc.threshold * P.a0;
-        }
+    if (trainSlot != ~0u) {
+        cc.b.trainContrib[trainSlot] = storeSpec<N>(P.contrib);
+        cc.b.trainAfterStamp[trainSlot] = cc.stamp;
     }
-    if (maxLengthTerminate) return;
-    P.rngUsed = true;
-    if (!cacheEnd) {
-        float continueProb = fminf(P.alpha.importance(P.wls.sel) / P.initImportance, 1.0f);
-        if (P.rng.uniform() >= continueProb) return;
-        P.alpha = P.alpha / continueProb;
-    }
-    Bsdf<N> bsdf = setupBsdf<N, NODES>(sc, mat, P.wls, &sp);
-    if (cacheEnd && cc.full) {
-        if (bsdf.hasNonDelta()) {
-            // the cache supplies all the radiance this vertex reflects; no next-event estimate
-            writeCacheRecord(sc, sp, G.material, rayDir, N == 4 ? P.wls.offset : 0.0f, cc.b.queryRaw + 4 * path);
-            cc.b.queryThroughput[path] = storeSpec<N>(P.alpha);
-            cc.b.queryStamp[path] = cc.stamp;
-            return;
-        }
-        // a purely specular vertex does not end in the cache: the path goes on
-        cacheEnd = false;
-        float continueProb = fminf(P.alpha.importance(P.wls.sel) / P.initImportance, 1.0f);
-        if (P.rng.uniform() >= continueProb) return;
-        P.alpha = P.alpha / continueProb;
-    }
-    V3 gnL = sp.frame.toLocal(sp.gn);
-    if (bsdf.hasNonDelta()) {
-        float uLight = P.rng.uniform();
-        float uP0 = P.rng.uniform(), uP1 = P.rng.uniform();
-        // a scene without emitters has nothing to sample (the draws are still made)
-        if (sc.lightInstIntegral > 0.0f) {
-            LightSample ls;
-            float lightProb;
-            sampleLight(sc, uLight, uP0, uP1, &ls, &lightProb);
-            const DevMaterial &lm = sc.materials[ls.material];
-            // shadow ray direction (SurfacePoint::calcDirectionFrom)
-            V3 sdir;
-            float dist2;
-            if (ls.sp.atInfinity) {
-                dist2 = 1.0f;
-                sdir = normalize(ls.sp.position);
-            } else {
-                V3 dv = ls.sp.position - sp.position;
-                dist2 = dv.sqLength();
-                sdir = dv / sqrtf(dist2);
-            }
-            V3 sdl = ls.sp.frame.toLocal(-sdir);
-            Spec<N> M;
-            float fe;
-            evalEDF<N, NODES>(sc, lm, ls.sp, P.wls, sdl, &M, &fe);
-            if (!M.isZero()) {
-                float rec = 1.0f / dist2;
-                V3 sdsn = sp.frame.toLocal(sdir);
-                float lightPDF = lightProb * ls.areaPDF;
-                Spec<N> fs = bsdf.evaluate(dirOutLocal, gnL, sdsn);
-                float cosLight = ls.sp.isPoint ? 1.0f : absDot(-sdir, ls.sp.gn);
-                float bsdfPDF = bsdf.evaluatePDF(dirOutLocal, sdsn, P.wls.sel) * cosLight * rec;
-                float mis = 1.0f;
-                if (!dt::isDelta(ls.posType) && !isinf(lightPDF))
-                    mis = (lightPDF * lightPDF) / (lightPDF * lightPDF + bsdfPDF * bsdfPDF);
-                float Gf = 1.0f * absDot(sdsn, gnL) * cosLight * rec;
-                float scalarCoeff = Gf * mis / lightPDF;
-                Spec<N> value = P.alpha * (M * fe) * fs * scalarCoeff;
-                // testVisibility (light_transport_common.h:147-177)
-                bool front = dot(sp.gn, sdir) > 0;
-                V3 so = offsetRayOrigin(sp.position, front ? sp.gn : -sp.gn);
-                front = -dot(ls.sp.gn, sdir) > 0;
-                V3 lo = offsetRayOrigin(ls.sp.position, front ? ls.sp.gn : -ls.sp.gn);
-                float tmax = 3.402823466e+38f;
-                if (!ls.sp.atInfinity) tmax = (lo - so).length() * 0.9999f;
-                *emitShadow = true;
-                *shOrg = make_float4(so.x, so.y, so.z, __uint_as_float(path));
-                *shDir = make_float4(sdir.x, sdir.y, sdir.z, tmax);
-                *shVal = storeSpec<N>(value);
-            }
-        }
+    if (!goesOn) return;
+    if (nextEvent && !M.isZero()) {
+        float rec = 1.0f / dist2;
+        V3 sdsn = sp.frame.toLocal(sdir);
+        float lightPDF = lightProb * ls.areaPDF;
+        float dirPDF;
+        Spec<N> fs = bsdf.evaluateWithPDF(dirOutLocal, gnL, sdsn, P.wls.sel, &dirPDF);
+        float cosLight = ls.sp.isPoint ? 1.0f : absDot(-sdir, ls.sp.gn);
+        float bsdfPDF = dirPDF * cosLight * rec;
+        float mis = 1.0f;
+        if (!dt::isDelta(ls.posType) && !isinf(lightPDF))
+            mis = (lightPDF * lightPDF) / (lightPDF * lightPDF + bsdfPDF * bsdfPDF);
+        float Gf = 1.0f * absDot(sdsn, gnL) * cosLight * rec;
+        float scalarCoeff = Gf * mis / lightPDF;
+        Spec<N> value = P.alpha * (M * fe) * fs * scalarCoeff;
+        // testVisibility (light_transport_common.h:147-177)
+        bool front = dot(sp.gn, sdir) > 0;
+        V3 so = offsetRayOrigin(sp.position, front ? sp.gn : -sp.gn);
+        front = -dot(ls.sp.gn, sdir) > 0;
+        V3 lo = offsetRayOrigin(ls.sp.position, front ? ls.sp.gn : -ls.sp.gn);
+        float tmax = 3.402823466e+38f;
+        if (!ls.sp.atInfinity) tmax = (lo - so).length() * 0.9999f;
+        *emitShadow = true;
+        *shOrg = make_float4(so.x, so.y, so.z, __uint_as_float(path));
+        *shDir = make_float4(sdir.x, sdir.y, sdir.z, tmax);
+        *shVal = storeSpec<N>(value);
     }
     if (cacheEnd) {
         // the cache supplies the indirect radiance leaving this vertex (what a continued path
         // would add after the next-event estimate above); the path ends here
-        writeCacheRecord(sc, sp, G.material, rayDir, N == 4 ? P.wls.offset : 0.0f, cc.b.queryRaw + 4 * path);
+        writeCacheRecord(sc, sp, sc.geomInsts[ha.y].material, rayDir, N == 4 ? P.wls.offset : 0.0f,
+                         cc.b.queryRaw + 4 * path);
         cc.b.queryThroughput[path] = storeSpec<N>(P.alpha);
         cc.b.queryStamp[path] = cc.stamp;
         return;

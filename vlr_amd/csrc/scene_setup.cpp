@@ -472,6 +472,9 @@ void buildSceneGPU(Context &ctx, const Scene &scene, bool spectral, SceneGPU *g)
     D.lightInstBase = static_cast<uint32_t>(pool.size());
     D.numLightInsts = static_cast<uint32_t>(lightImp.size());
     D.lightInstIntegral = appendDiscrete(pool, lightImp);
+    D.numLightInstsSearched = D.numLightInsts;
+    const float *lightCdf = pool.data() + D.lightInstBase + D.numLightInsts;
+    while (D.numLightInstsSearched > 1 && lightCdf[D.numLightInstsSearched - 1] == 1.0f) --D.numLightInstsSearched;
 
     // scene bounds (setup_scene.cu:82-92)
     if (!sceneBox.empty()) {

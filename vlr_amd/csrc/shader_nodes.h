@@ -455,8 +455,8 @@ __device__ __forceinline__ void materialNodes(const DevScene &sc, const DevMater
 
 template <int N>
 __device__ __forceinline__ Spec<N> materialSpectrum(const DevScene &sc, const DevMaterial &m, int k,
-                                                    const NodeOutputs<N> &o, const Wls<N> &wls) {
-    return (o.has & (1u << k)) ? o.spec[k] : evalSpectrum<N>(sc, m.spec[k], wls);
+                                                    const NodeOutputs<N> &o, const SpecBins<N> &bins) {
+    return (o.has & (1u << k)) ? o.spec[k] : evalSpectrum<N>(sc, m.spec[k], bins);
 }
 
 // GGX alphas and rotation from roughness / anisotropy / rotation (materials.cu:1230-1236)
@@ -468,66 +468,44 @@ __device__ __forceinline__ void ggxParams(const float4 &rar, float *ax, float *a
     *rot = 2 * kPiF * rar.z;
 }
 
-// Material set-up at a surface point (the *_setupBSDF callables of materials.cu)
+// Material set-up at a surface point (the *_setupBSDF callables of materials.cu).  The material's
+// spectra are evaluated before the types part, so that lanes of different types do it together.
 template <int N, bool NODES = true>
 __device__ __forceinline__ Bsdf<N> setupBsdf(const DevScene &sc, const DevMaterial &m, const Wls<N> &wls,
-                                             const SurfPt *sp) {
+                                             const SpecBins<N> &bins, const SurfPt *sp) {
     NodeOutputs<N> o;
     if constexpr (NODES) materialNodes<N>(sc, m, sp, wls, &o);
     else o.has = 0;
+    // per type: its BSDF (four bits) and number of spectra (two bits)
+    constexpr uint64_t kKinds = (uint64_t(BSDF_MATTE) << 4 * MAT_MATTE) |
+                                (uint64_t(BSDF_SPEC_BRDF) << 4 * MAT_SPECULAR_REFLECTION) |
+                                (uint64_t(BSDF_SPEC_BSDF) << 4 * MAT_SPECULAR_SCATTERING) |
+                                (uint64_t(BSDF_MICRO_BRDF) << 4 * MAT_MICROFACET_REFLECTION) |
+                                (uint64_t(BSDF_DIFFSPEC) << 4 * MAT_UE4) |
+                                (uint64_t(BSDF_MICRO_BSDF) << 4 * MAT_MICROFACET_SCATTERING);
+    constexpr uint32_t kSpectra = (1u << 2 * MAT_MATTE) | (3u << 2 * MAT_SPECULAR_REFLECTION) |
+                                  (3u << 2 * MAT_SPECULAR_SCATTERING) | (2u << 2 * MAT_MICROFACET_REFLECTION) |
+                                  (1u << 2 * MAT_UE4) | (3u << 2 * MAT_MICROFACET_SCATTERING);
+    const uint32_t type = m.type, spectra = (kSpectra >> (2 * type)) & 3u;
     Bsdf<N> b;
-    b.kind = BSDF_NULL;
-    b.a0 = b.a1 = b.a2 = 0.0f;
-    b.dispersive = false;
-    switch (m.type) {
-    case MAT_MATTE:
-        b.kind = BSDF_MATTE;
-        b.c0 = materialSpectrum<N>(sc, m, 0, o, wls);
-        break;
-    case MAT_SPECULAR_REFLECTION:
-        b.kind = BSDF_SPEC_BRDF;
-        b.c0 = materialSpectrum<N>(sc, m, 0, o, wls);
-        b.c1 = materialSpectrum<N>(sc, m, 1, o, wls);
-        b.c2 = materialSpectrum<N>(sc, m, 2, o, wls);
-        break;
-    case MAT_SPECULAR_SCATTERING:
-        b.kind = BSDF_SPEC_BSDF;
-        b.c0 = materialSpectrum<N>(sc, m, 0, o, wls);
-        b.c1 = materialSpectrum<N>(sc, m, 1, o, wls);
-        b.c2 = materialSpectrum<N>(sc, m, 2, o, wls);
-        b.dispersive = !wls.single;
-        break;
-    case MAT_MICROFACET_REFLECTION:
-        // materials.cu:1226-1236; alphas derived on the host unless a node supplies the parameters
-        b.kind = BSDF_MICRO_BRDF;
-        b.c0 = materialSpectrum<N>(sc, m, 0, o, wls);
-        b.c1 = materialSpectrum<N>(sc, m, 1, o, wls);
-        if (o.has & 8u) {
-            ggxParams(o.vec[0], &b.a0, &b.a1, &b.a2);
-        } else {
-            b.a0 = m.scalars[0];
-            b.a1 = m.scalars[1];
-            b.a2 = m.scalars[2];
-        }
-        break;
-    case MAT_MICROFACET_SCATTERING:
-        // materials.cu:1516-1536
-        b.kind = BSDF_MICRO_BSDF;
-        b.c0 = materialSpectrum<N>(sc, m, 0, o, wls);
-        b.c1 = materialSpectrum<N>(sc, m, 1, o, wls);
-        b.c2 = materialSpectrum<N>(sc, m, 2, o, wls);
-        if (o.has & 8u) {
-            ggxParams(o.vec[0], &b.a0, &b.a1, &b.a2);
-        } else {
-            b.a0 = m.scalars[0];
-            b.a1 = m.scalars[1];
-            b.a2 = m.scalars[2];
-        }
-        break;
-    case MAT_UE4: {
+    b.kind = static_cast<uint32_t>(kKinds >> (4 * type)) & 15u;
+    b.dispersive = type == MAT_SPECULAR_SCATTERING && !wls.single;
+    b.c0 = b.c1 = b.c2 = Spec<N>(0.0f);
+    if (spectra > 0) b.c0 = materialSpectrum<N>(sc, m, 0, o, bins);
+    if (spectra > 1) b.c1 = materialSpectrum<N>(sc, m, 1, o, bins);
+    if (spectra > 2) b.c2 = materialSpectrum<N>(sc, m, 2, o, bins);
+    // microfacet types (materials.cu:1226-1236, 1516-1536): alphas and rotation, derived on the host
+    // unless a node supplies the parameters.  (No switch with these two types sharing a case: its
+    // gfx950 code lost the first of the three for one of them.)
+    const bool micro = type == MAT_MICROFACET_REFLECTION || type == MAT_MICROFACET_SCATTERING;
+    float ax = m.scalars[0], ay = m.scalars[1], rotation = m.scalars[2];
+    if (micro && (o.has & 8u)) ggxParams(o.vec[0], &ax, &ay, &rotation);
+    b.a0 = micro ? ax : 0.0f;
+    b.a1 = micro ? ay : 0.0f;
+    b.a2 = micro ? rotation : 0.0f;
+    if (type == MAT_UE4) {
         // materials.cu:1959-1978
-        b.kind = BSDF_DIFFSPEC;
-        Spec<N> base = materialSpectrum<N>(sc, m, 0, o, wls);
+        const Spec<N> base = b.c0;
         float roughness = m.scalars[1], metallic = m.scalars[2];
         if (o.has & 8u) {
             roughness = o.vec[0].y;
@@ -538,12 +516,13 @@ __device__ __forceinline__ Bsdf<N> setupBsdf(const DevScene &sc, const DevMateri
         b.c0 = base * (1 - metallic);
         b.c1 = lerpSpec<N>(Spec<N>(0.08f * specular), base, metallic);
         b.a0 = roughness;
-        break;
-    }
-    default:
-        break;
     }
     return b;
+}
+template <int N, bool NODES = true>
+__device__ __forceinline__ Bsdf<N> setupBsdf(const DevScene &sc, const DevMaterial &m, const Wls<N> &wls,
+                                             const SurfPt *sp) {
+    return setupBsdf<N, NODES>(sc, m, wls, SpecBins<N>(wls), sp);
 }
 
 } // namespace vlra
