@@ -236,6 +236,7 @@ struct DevScene {
     const float* nodePool;        // sampled-spectrum tables of nodes
     uint32_t numInstances;
     uint32_t hasTlas;
+    uint32_t numTriangles;       // in the bottom-level trees, each counted once
     uint32_t hasNodePrograms;    // some material or material group has a node program
     uint32_t hasAlpha;           // some triangle group has an alpha node (stochastic alpha test)
     // light selection over [environment, instances...]

@@ -207,15 +207,18 @@ struct TravCount {
 
 typedef int32_t StackPair __attribute__((ext_vector_type(2)));   // node code, entry distance
 
-// Traversal state: one ray's walk through the two-level BVH.  The node stack
-// lives in LDS (kLdsStack entries per lane) with an overflow area the caller keeps in scratch.
+// Traversal state: one ray's walk through the two-level BVH.  The node stack lives in LDS
+// (kLdsStack entries per lane) with an overflow area in scratch, its top entry in registers.
 constexpr int32_t kTravDone = INT32_MIN + 1;
 struct TravState {
     V3 org, dir;                  // the world-space ray
     RayPre ray;                   // in the space of the tree being walked
     float tmin, tmax;
     int32_t cur, curInst;
-    int sp, spBlas;               // stack height, and the height at which the instance was entered
+    int32_t topCode;              // walkTop: the stack's top entry; kTravDone below all others,
+    float topT;                   // kSentinel below an instance's
+    int sp;                       // entries in LDS and scratch
+    int spBlas;                   // walkLds: their number at which the instance was entered
     const BVH4QNode *nodes;       // the tree being walked
     const TriRecord *tris;
     bool inBlas, found;
@@ -235,45 +238,291 @@ __device__ __forceinline__ void travBegin(TravState &st, const DevScene &sc, con
     st.ray.init(org, dir);
     st.tmin = tmin;
     st.tmax = tmax;
-    st.cur = sc.hasTlas ? 0 : kTravDone;
     st.curInst = -1;
-    st.sp = st.spBlas = 0;
     st.nodes = sc.tlasNodes;
     st.tris = sc.blasTris;
-    st.inBlas = false;
-    st.found = false;
     st.hit.inst = -1;
     st.hit.geomInst = st.hit.prim = -1;
     st.hit.t = st.hit.b1 = st.hit.b2 = 0.0f;
     st.rng = nullptr;
+    st.inBlas = false;
+    st.found = false;
     st.vis = 1.0f;
 }
 
-// Runs the traversal to its end (then st.found and st.hit hold the closest hit, or any hit for
-// an any-hit ray).  The loop is a while-while loop: a lane walks inner nodes until it reaches a
-// leaf, an instance's end or the end of the walk, and only then handles that one item
-// (enter the instance, test the leaf's triangles, or leave the instance) before walking inner
-// nodes again.  Each lane visits the same nodes in the same order as a one-item-per-iteration
-// loop; the wave just runs its lanes' inner-node visits together and their leaves together.
-// With ALPHA, triangles of groups with an alpha node pass the stochastic alpha test
-// (path_tracing.cu:14-25) for closest-hit rays and scale the fractional visibility
-// (light_transport_common.h:205-218) for any-hit rays.
-// ANY: an any-hit ray, which needs no visiting order: its children are stacked as they come,
-// without entry distances.
-// SD: stack entries per lane in LDS, (code, entry distance) pairs of which an any-hit ray uses the
-// codes; the other kTravStackCapacity - SD entries are in ovf.  A lane's entries have the same
-// places for both kinds of rays, because the waves of a block run the two at the same time.  CODES:
-// places for codes only, in a kernel that traces nothing but any-hit rays.
-template <bool ANY, bool STATS, bool ALPHA = false, int SD = kLdsStack, bool CODES = false>
-__device__ __forceinline__ void traverse(TravState &st, const DevScene &sc, int32_t *ldsWords, int lane,
-                                         TravCount *tc) {
+// Stack entries below the top: SD per lane in LDS, (code, entry distance) pairs of which an any-hit
+// ray uses the codes, and the others in scratch.  A lane's entries have the same places for both
+// kinds of rays, because the waves of a block run the two at the same time.  CODES: places for codes
+// only, in a kernel that traces nothing but any-hit rays.
+// Each entry keeps the distance at which the ray enters its box; once a closer hit has shrunk tmax
+// past it (widened by 8 ulps), the entry is dropped unvisited.  Scene set-up bounds the depth by
+// kTravStackCapacity (travStackBound, to which the entries below the two trees' roots add), so the index never
+// reaches past the scratch area; the clamp only keeps the access inside the array.  The LDS part is
+// addressed as LDS: with generic pointers the two parts' accesses merge into flat ones, which wait
+// for every memory counter.
+template <bool ANY, int SD, bool CODES>
+struct TravStack {
+    static_assert(ANY || !CODES, "closest-hit rays keep entry distances");
+    using Entry = std::conditional_t<ANY, int32_t, StackPair>;
+    using Lds = __attribute__((address_space(3))) Entry *;
+    static constexpr int kOvf = static_cast<int>(kTravStackCapacity) + 2 - SD;
+    static constexpr int kStride = kTraceBlock * (ANY && !CODES ? 2 : 1);   // between a lane's entries
+    static __device__ __forceinline__ Lds column(int32_t *words, int lane) {
+        return (Lds)words + lane * (kStride / kTraceBlock);
+    }
+    static __device__ __forceinline__ Entry entry(int32_t v, float t) {
+        if constexpr (ANY) return v;
+        else return StackPair{v, __float_as_int(t)};
+    }
+    static __device__ __forceinline__ void store(Lds lds, Entry *ovf, int at, int32_t v, float t) {
+        if (at < SD) lds[at * kStride] = entry(v, t);
+        else ovf[min(at - SD, kOvf - 1)] = entry(v, t);
+    }
+    // the walk starts at the root of the top-level tree (entry 0 is what the last pop loads in the
+    // top's place)
+    static __device__ __forceinline__ void start(TravState &st, const DevScene &sc) {
+        st.cur = sc.hasTlas ? 0 : kTravDone;
+        st.topCode = kTravDone;
+        st.topT = -__builtin_huge_valf();
+        st.sp = 1;
+    }
+    static __device__ __forceinline__ void push(Lds lds, Entry *ovf, TravState &st, int32_t v, float t) {
+        store(lds, ovf, st.sp, st.topCode, st.topT);
+        ++st.sp;
+        st.topCode = v;
+        st.topT = t;
+    }
+    // The top entry becomes the current node, dropping entries that lie beyond the closest hit so far
+    // (an any-hit ray stops at its first hit, so every entry it pops is still open), and the next one
+    // is loaded in its place, to be there by the next pop.
+    static __device__ __forceinline__ void pop(Lds lds, Entry *ovf, TravState &st) {
+        const float tCull = st.tmax * (1.0f + 8.0f * __FLT_EPSILON__);
+        bool drop;
+        do {
+            st.cur = st.topCode;
+            drop = !ANY && st.topT > tCull;
+            --st.sp;
+            Entry e;
+            if (st.sp < SD) e = lds[st.sp * kStride];
+            else e = ovf[min(st.sp - SD, kOvf - 1)];
+            if constexpr (ANY) {
+                st.topCode = e;
+            } else {
+                st.topCode = e.x;
+                st.topT = __int_as_float(e.y);
+            }
+        } while (drop);
+    }
+};
+
+// Visits the inner node st.cur and moves on to its nearest child that the ray meets, or to the
+// next stack entry.  ANY: an any-hit ray, which needs no visiting order: its children are stacked
+// as they come, without entry distances.
+template <bool ANY, int SD, bool CODES>
+__device__ __forceinline__ void innerStep(TravState &st, typename TravStack<ANY, SD, CODES>::Lds lds,
+                                          typename TravStack<ANY, SD, CODES>::Entry *ovf) {
+    using Stack = TravStack<ANY, SD, CODES>;
+    const uint4 *np = reinterpret_cast<const uint4 *>(st.nodes + st.cur);
+    const uint4 w0 = np[0], w1 = np[1], w2 = np[2];
+    const uint2 w3 = *reinterpret_cast<const uint2 *>(np + 3);
+    const RayPre &r = st.ray;
+    // step = 2^(e - 127) per axis
+    const NodeAxis X(__uint_as_float(w0.x), __uint_as_float((w0.w << 23) & 0x7F800000u), r.inv.x, r.oi.x),
+        Y(__uint_as_float(w0.y), __uint_as_float((w0.w << 15) & 0x7F800000u), r.inv.y, r.oi.y),
+        Z(__uint_as_float(w0.z), __uint_as_float((w0.w << 7) & 0x7F800000u), r.inv.z, r.oi.z);
+    const bool nx = r.inv.x < 0.0f, ny = r.inv.y < 0.0f, nz = r.inv.z < 0.0f;
+    const uint32_t qnx = nx ? w1.w : w1.x, qfx = nx ? w1.x : w1.w;
+    const uint32_t qny = ny ? w2.x : w1.y, qfy = ny ? w1.y : w2.x;
+    const uint32_t qnz = nz ? w2.y : w1.z, qfz = nz ? w1.z : w2.y;
+    const float tmaxWide = st.tmax * (1.0f + 8.0f * __FLT_EPSILON__);
+    constexpr float kMiss = __builtin_huge_valf();
+    // entry distance of child k, or kMiss; child code 0 (the root's index) marks an empty slot
+    auto enter = [&](int k, int32_t c) {
+        auto q = [&](uint32_t w) { return static_cast<float>((w >> (8 * k)) & 0xFFu); };
+        const float tn = fmaxf(fmaxf(fmaxf(__builtin_fmaf(q(qnx), X.a, X.bNear), __builtin_fmaf(q(qny), Y.a, Y.bNear)),
+                                     __builtin_fmaf(q(qnz), Z.a, Z.bNear)), st.tmin);
+        const float tf = fminf(fminf(__builtin_fmaf(q(qfx), X.a, X.bFar), __builtin_fmaf(q(qfy), Y.a, Y.bFar)),
+                               __builtin_fmaf(q(qfz), Z.a, Z.bFar));
+        return (c != 0) & (tn <= fminf(tf, tmaxWide)) ? tn : kMiss;
+    };
+    int32_t c0 = static_cast<int32_t>(w2.z), c1 = static_cast<int32_t>(w2.w), c2 = static_cast<int32_t>(w3.x),
+            c3 = static_cast<int32_t>(w3.y);
+    float t0 = enter(0, c0), t1 = enter(1, c1), t2 = enter(2, c2), t3 = enter(3, c3);
+    if constexpr (ANY) {
+        // any order will do: stack the hit children but the first, visit that one next
+        int32_t next = 0;   // 0 is never a child code
+        auto take = [&](int32_t c, float t) {
+            const bool hit = t != kMiss;
+            if (hit && next != 0) Stack::push(lds, ovf, st, c, t);
+            next = hit && next == 0 ? c : next;
+        };
+        take(c0, t0);
+        take(c1, t1);
+        take(c2, t2);
+        take(c3, t3);
+        st.cur = next;
+        if (next == 0) Stack::pop(lds, ovf, st);
+    } else {
+        // sort the four (distance, child) pairs, nearest first; misses sort last
+        auto cswap = [](float &ta, int32_t &ca, float &tb, int32_t &cb) {
+            const bool s = tb < ta;
+            const float tl = s ? tb : ta, th = s ? ta : tb;
+            const int32_t cl = s ? cb : ca, ch = s ? ca : cb;
+            ta = tl; tb = th;
+            ca = cl; cb = ch;
+        };
+        cswap(t0, c0, t1, c1);
+        cswap(t2, c2, t3, c3);
+        cswap(t0, c0, t2, c2);
+        cswap(t1, c1, t3, c3);
+        cswap(t1, c1, t2, c2);
+        const bool h1 = t1 != kMiss, h2 = t2 != kMiss, h3 = t3 != kMiss;
+        if (st.sp + 3 <= SD) {
+            // the old top, c3 and c2 go to consecutive places, what is not stacked being overwritten
+            auto *at = lds + st.sp * Stack::kStride;
+            at[0] = Stack::entry(st.topCode, st.topT);
+            at += h1 ? Stack::kStride : 0;
+            at[0] = Stack::entry(c3, t3);
+            at += h3 ? Stack::kStride : 0;
+            at[0] = Stack::entry(c2, t2);
+            st.sp += static_cast<int>(h1) + static_cast<int>(h2) + static_cast<int>(h3);
+            st.topCode = h1 ? c1 : st.topCode;
+            st.topT = h1 ? t1 : st.topT;
+        } else {
+            if (h3) Stack::push(lds, ovf, st, c3, t3);
+            if (h2) Stack::push(lds, ovf, st, c2, t2);
+            if (h1) Stack::push(lds, ovf, st, c1, t1);
+        }
+        st.cur = c0;
+        if (t0 == kMiss) Stack::pop(lds, ovf, st);
+    }
+}
+
+// Tests the triangles of the leaf st.cur of an instance; returns true when an any-hit ray is
+// blocked.  The next triangle's record is loaded while one is tested.  With ALPHA, triangles of
+// groups with an alpha node pass the stochastic alpha test (path_tracing.cu:14-25) for closest-hit
+// rays and scale the fractional visibility (light_transport_common.h:205-218) for any-hit rays.
+template <bool ALPHA>
+__device__ __forceinline__ bool leafStep(TravState &st, const DevScene &sc, bool anyHit) {
+    const uint32_t code = ~static_cast<uint32_t>(st.cur);
+    const uint32_t last = code & (kMaxLeafPrims - 1);
+    const float4 *tp = reinterpret_cast<const float4 *>(st.tris + (code >> kLeafShift));
+    float4 n0 = tp[0], n1 = tp[1], n2 = tp[2];
+    for (uint32_t k = 0;; ++k) {
+        const float4 q0 = n0, q1 = n1, q2 = n2;
+        if (k < last) {
+            tp += 3;
+            n0 = tp[0];
+            n1 = tp[1];
+            n2 = tp[2];
+        }
+        float t, b1, b2;
+        bool hit = intersectTri(st.ray, xyz(q0), xyz(q1), xyz(q2), st.tmin, st.tmax, &t, &b1, &b2);
+        if constexpr (ALPHA) {
+            const uint32_t gi = __float_as_uint(q0.w);
+            if (hit && sc.hasAlpha && sc.geomInsts[gi].alphaCount) {
+                const float alpha = alphaAt(sc, st.curInst, gi, __float_as_uint(q1.w), b1, b2);
+                if (anyHit) {
+                    st.vis *= 1 - alpha;
+                    hit = st.vis == 0.0f;
+                } else if (st.rng) {
+                    hit = !(st.rng->uniform() >= alpha);
+                }
+            }
+        }
+        if (hit) {
+            st.tmax = t;
+            st.found = true;
+            st.hit.inst = st.curInst;
+            st.hit.geomInst = static_cast<int32_t>(__float_as_uint(q0.w));
+            st.hit.prim = static_cast<int32_t>(__float_as_uint(q1.w));
+            st.hit.b1 = b1;
+            st.hit.b2 = b2;
+            if (anyHit) return true;
+        }
+        if (k == last) return false;
+    }
+}
+
+// With st.cur a leaf of the top-level tree: the walk enters that instance.  Otherwise (an inner
+// node of the top-level tree) it goes on there.  Sets the tree and the ray of the space it is in.
+template <typename Stack>
+__device__ __forceinline__ void spaceStep(TravState &st, const DevScene &sc, typename Stack::Lds lds,
+                                          typename Stack::Entry *ovf) {
+    V3 o = st.org, d = st.dir;
+    if (st.cur < 0) {
+        st.curInst = static_cast<int32_t>((~static_cast<uint32_t>(st.cur)) >> kLeafShift);
+        const DevInstance &I = sc.instances[st.curInst];
+        o = xfmPoint(I.w2o, st.org);
+        d = xfmVector(I.w2o, st.dir);
+        st.nodes = sc.blasNodes + I.blasNodeBase;
+        st.tris = sc.blasTris + I.blasTriBase;
+        st.inBlas = true;
+        Stack::push(lds, ovf, st, kSentinel, -__builtin_huge_valf());
+        st.cur = 0;
+    } else {
+        st.nodes = sc.tlasNodes;
+    }
+    st.ray.init(o, d);
+}
+
+// Two walks, visiting the same nodes in the same order, each to its end (then st.found and st.hit hold
+// the closest hit, or any hit for an any-hit ray).  Both are while-while loops: a lane walks inner
+// nodes until it reaches a leaf, an instance's end or the end of the walk, and only then handles that
+// one item (enter the instance, test the leaf's triangles, or leave the instance) before walking inner
+// nodes again.  The wave so runs its lanes' inner-node visits together and their leaves together.
+//
+// walkTop keeps the stack's top entry in registers, so that the node after a miss is known before
+// the LDS is read, and loads a leaf's next triangle while it tests one; walkLds keeps neither.
+// Measured, walkLds / walkTop: 2^21 incoherent rays in the icosphere grid 1.77 / 1.40 ms, its 1080p
+// frames 26.3 / 22.8 ms (8), 270 k triangles at 641 x 427 3.86 / 3.45 ms (4), a batch of 24 jobs
+// 33.9 / 33.0 ms.  The kernels that spill in any case lose by the registers more than they gain:
+// LVC-BPT 720p 6.64 / 6.93 ms, light tracing 720p 3.46 / 3.60 ms, and the tail kernel with node
+// programs (textured 720p 3.74 / 3.81 ms); they use walkLds.  So does the tail kernel where the walks
+// are too short for the top entry to matter (fewer than kTopWalkTriangles in the scene): the Cornell
+// box of 36 triangles at 256 x 256 takes 4.50 / 4.67 ms (16), 160 x 90 previews of it 262 / 269 us.
+constexpr uint32_t kTopWalkTriangles = 4096;
+template <bool ANY, bool STATS, bool ALPHA, int SD, bool CODES>
+__device__ __forceinline__ void walkTop(TravState &st, const DevScene &sc, int32_t *ldsWords, int lane,
+                                        TravCount *tc) {
+    using Stack = TravStack<ANY, SD, CODES>;
+    const typename Stack::Lds lds = Stack::column(ldsWords, lane);
+    typename Stack::Entry ovf[Stack::kOvf];
+    Stack::start(st, sc);
+    while (st.cur != kTravDone) {
+        while (st.cur >= 0) {
+            if constexpr (STATS) ++tc->nodes;
+            innerStep<ANY, SD, CODES>(st, lds, ovf);
+        }
+        if (st.cur == kTravDone) break;
+        if (st.inBlas && st.cur != kSentinel) {
+            if constexpr (STATS) tc->tris += ((~static_cast<uint32_t>(st.cur)) & (kMaxLeafPrims - 1)) + 1;
+            if (leafStep<ALPHA>(st, sc, ANY)) break;
+            Stack::pop(lds, ovf, st);
+            continue;
+        }
+        // Leave the instance (kSentinel), enter the next one (a leaf of the top-level tree), or
+        // both: the ray is set up once for the space the walk goes on in.
+        if (st.cur == kSentinel) {
+            st.inBlas = false;
+            Stack::pop(lds, ovf, st);
+            if (st.cur == kTravDone) break;
+        }
+        if constexpr (STATS) tc->insts += st.cur < 0;
+        spaceStep<Stack>(st, sc, lds, ovf);
+    }
+    st.hit.t = st.tmax;
+}
+
+// rng: the path's generator (closest-hit rays through alpha surfaces); vis: the fractional
+// visibility of an any-hit ray (0 when occluded)
+template <bool ANY, bool STATS, bool ALPHA, int SD, bool CODES>
+__device__ __forceinline__ void walkLds(TravState &st, const DevScene &sc, int32_t *ldsWords, int lane,
+                                        TravCount *tc) {
     constexpr int kOvf = static_cast<int>(kTravStackCapacity) - SD;
-    // each stack entry keeps the distance at which the ray enters its box; once a closer hit
-    // has shrunk tmax past it (widened by 8 ulps), the entry is dropped unvisited.
-    // Scene set-up bounds the depth by kTravStackCapacity (travStackBound), so the index never
-    // reaches past the scratch area; the clamp only keeps the access inside the array.
-    // The LDS part is addressed as LDS: with generic pointers the two parts' accesses merge into
-    // flat ones, which wait for every memory counter.
+    st.cur = sc.hasTlas ? 0 : kTravDone;
+    st.sp = st.spBlas = 0;
+    // entries as in TravStack, all of them in LDS and scratch
     using Entry = std::conditional_t<ANY, int32_t, StackPair>;
     static_assert(ANY || !CODES, "closest-hit rays keep entry distances");
     constexpr int kStride = kTraceBlock * (ANY && !CODES ? 2 : 1);   // from one entry of a lane to the next
@@ -451,14 +700,15 @@ __device__ __forceinline__ void traverse(TravState &st, const DevScene &sc, int3
 
 // rng: the path's generator (closest-hit rays through alpha surfaces); vis: the fractional
 // visibility of an any-hit ray (0 when occluded)
-template <bool ANY, bool STATS = false, bool ALPHA = false, int SD = kLdsStack, bool CODES = false>
+template <bool ANY, bool STATS = false, bool ALPHA = false, int SD = kLdsStack, bool CODES = false, bool TOP = true>
 __device__ __forceinline__ bool traceRay(const DevScene &sc, const V3 &org, const V3 &dir, float tmin, float tmax,
                                          TraceHit *hit, int32_t *lds, int lane, TravCount *tc = nullptr,
                                          Pcg32 *rng = nullptr, float *vis = nullptr) {
     TravState st;
     travBegin(st, sc, org, dir, tmin, tmax);
     st.rng = rng;
-    traverse<ANY, STATS, ALPHA, SD, CODES>(st, sc, lds, lane, tc);
+    if constexpr (TOP) walkTop<ANY, STATS, ALPHA, SD, CODES>(st, sc, lds, lane, tc);
+    else walkLds<ANY, STATS, ALPHA, SD, CODES>(st, sc, lds, lane, tc);
     if (st.found) *hit = st.hit;
     if (vis) *vis = st.found ? 0.0f : st.vis;
     return st.found;
@@ -1097,7 +1347,8 @@ struct PathRegs {
     float a0, a;    // radiance cache: path spread at the first vertex and accumulated since
 };
 
-template <int N>
+// CACHE: the radiance cache may be on (CacheCtx::mode says whether it is)
+template <int N, bool CACHE = true>
 __device__ __forceinline__ void loadPath(const FrameBuffers &fb, uint32_t path, PathRegs<N> *P) {
     P->alpha = loadSpec<N>(fb.ps.alpha[path]);
     P->contrib = loadSpec<N>(fb.ps.contrib[path]);
@@ -1112,7 +1363,7 @@ __device__ __forceinline__ void loadPath(const FrameBuffers &fb, uint32_t path, 
     P->rng.s = fb.ps.rng[path];
     P->rngUsed = false;
     P->a0 = P->a = 0.0f;
-    if (fb.cache.spread) {
+    if (CACHE && fb.cache.spread) {
         float2 sp = fb.cache.spread[path];
         P->a0 = sp.x;
         P->a = sp.y;
@@ -1169,7 +1420,7 @@ __device__ __forceinline__ void writeCacheRecord(const DevScene &sc, const SurfP
 // A wave's lanes miss, hit emitters and hit surfaces at once, and each kind needs some emitter's
 // emittance (the environment's, its own, the sampled light's): it is evaluated in one place for all
 // of them, as are the spectra of the materials (setupBsdf), in place of once per kind.
-template <int N, bool NODES = true>
+template <int N, bool NODES = true, bool CACHE = true>
 __device__ __forceinline__ void shadeStep(const DevScene &sc, uint32_t pathLength, uint32_t maxPathLength,
                                           uint32_t path, const V3 &rayOrg, const V3 &rayDir, int4 ha, float2 hb,
                                           PathRegs<N> &P, const CacheCtx &cc, bool *emitShadow, float4 *shOrg,
@@ -1178,7 +1429,7 @@ __device__ __forceinline__ void shadeStep(const DevScene &sc, uint32_t pathLengt
     *emitShadow = false;
     *emitNext = false;
     const bool maxLengthTerminate = pathLength >= maxPathLength;
-    if (cc.mode != 0 && !cc.full && pathLength >= 2 && pathLength - 1 <= kCacheTrainVerts) {
+    if (CACHE && cc.mode != 0 && !cc.full && pathLength >= 2 && pathLength - 1 <= kCacheTrainVerts) {
         // training path: the contribution before this vertex's emission closes the previous
         // vertex's sample (everything it gathered up to and including its next-event estimate)
         const uint32_t pix = (path / cc.width) * cc.imageW + path % cc.width;
@@ -1230,7 +1481,7 @@ __device__ __forceinline__ void shadeStep(const DevScene &sc, uint32_t pathLengt
             emitDir = dirOutLocal;
             emission = true;
         }
-        if (cc.mode != 0) {
+        if (CACHE && cc.mode != 0) {
             // path spread (Mueller et al. 2021, "Real-time Neural Radiance Caching for Path
             // Tracing"): a_0 from the primary vertex, then one term per non-delta bounce
             const float d2 = (sp.position - rayOrg).sqLength();
@@ -1269,7 +1520,7 @@ __device__ __forceinline__ void shadeStep(const DevScene &sc, uint32_t pathLengt
         }
         if (goesOn) {
             bsdf = setupBsdf<N, NODES>(sc, mat, P.wls, bins, &sp);
-            if (cacheEnd && cc.full) {
+            if (CACHE && cacheEnd && cc.full) {
                 if (bsdf.hasNonDelta()) {
                     // the cache supplies all the radiance this vertex reflects; no next-event estimate
                     writeCacheRecord(sc, sp, G.material, rayDir, N == 4 ? P.wls.offset : 0.0f, cc.b.queryRaw + 4 * path);
@@ -1329,7 +1580,7 @@ __device__ __forceinline__ void shadeStep(const DevScene &sc, uint32_t pathLengt
         }
         P.contrib += alphaIn * (M * fe) * mis;
     }
-    if (trainSlot != ~0u) {
+    if (CACHE && trainSlot != ~0u) {
         cc.b.trainContrib[trainSlot] = storeSpec<N>(P.contrib);
         cc.b.trainAfterStamp[trainSlot] = cc.stamp;
     }
@@ -1360,7 +1611,7 @@ __device__ __forceinline__ void shadeStep(const DevScene &sc, uint32_t pathLengt
         *shDir = make_float4(sdir.x, sdir.y, sdir.z, tmax);
         *shVal = storeSpec<N>(value);
     }
-    if (cacheEnd) {
+    if (CACHE && cacheEnd) {
         // the cache supplies the indirect radiance leaving this vertex (what a continued path
         // would add after the next-event estimate above); the path ends here
         writeCacheRecord(sc, sp, sc.geomInsts[ha.y].material, rayDir, N == 4 ? P.wls.offset : 0.0f,
@@ -1390,7 +1641,7 @@ __device__ __forceinline__ void shadeStep(const DevScene &sc, uint32_t pathLengt
     P.prevType = sType;
 }
 
-template <int N>
+template <int N, bool CACHE = true>
 __device__ __forceinline__ void storePath(const FrameBuffers &fb, uint32_t path, uint32_t pathLength,
                                           const PathRegs<N> &P, bool continues) {
     fb.ps.contrib[path] = storeSpec<N>(P.contrib);
@@ -1399,7 +1650,7 @@ __device__ __forceinline__ void storePath(const FrameBuffers &fb, uint32_t path,
         fb.ps.alpha[path] = storeSpec<N>(P.alpha);
         fb.ps.meta[path] = make_float4(P.wls.offset, P.prevDirPDF, P.initImportance,
                                        __uint_as_float(packFlags(P.wls.sel, P.wls.single, P.prevType, pathLength)));
-        if (fb.cache.spread) fb.cache.spread[path] = make_float2(P.a0, P.a);
+        if (CACHE && fb.cache.spread) fb.cache.spread[path] = make_float2(P.a0, P.a);
     }
 }
 
@@ -1566,7 +1817,9 @@ __global__ void __launch_bounds__(kTraceBlock) k_shadow(KArgs a) {
 // random numbers and adds its contributions in the same order as the per-depth kernels, so a
 // frame's result does not depend on the depth at which paths switch to this kernel.  Rays per
 // depth are counted in LDS and added to the frame counters once per block.
-template <int N, bool STATS, bool MULTI = false, bool NODES = true>
+// CACHE: the radiance cache may be on; without it its context and the path's spread take no registers
+// (textured 720p 3.86 / 3.60 ms, 4 frames).  TOP: which walk (walkTop or walkLds) its rays take.
+template <int N, bool STATS, bool MULTI = false, bool NODES = true, bool CACHE = true, bool TOP = false>
 __global__ void __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(kTailWavesPerEU)))
 k_tail(KArgs a) {
     __shared__ __attribute__((aligned(8))) int32_t lds[kTraceLds];
@@ -1575,7 +1828,8 @@ k_tail(KArgs a) {
     const uint32_t depth0 = a.depth;
     const uint32_t count = a.fb.counters[2 * depth0];
     const RayQueue q = a.fb.rays[depth0 & 1];
-    const CacheCtx cc = cacheCtx(a.fp, a.fb);
+    CacheCtx cc;
+    if constexpr (CACHE) cc = cacheCtx(a.fp, a.fb);
     for (uint32_t k = threadIdx.x; k < 2 * kMaxDepthCounters; k += blockDim.x) depthCounts[k] = 0;
     __syncthreads();
     TravCount tc, tcShadow;
@@ -1601,7 +1855,7 @@ k_tail(KArgs a) {
                         const float4 o4 = q.org[i], d4 = q.dir[i];
                         path = __float_as_uint(o4.w);
                         if constexpr (MULTI) job = jobOf(a, path);
-                        loadPath<N>(a.fb, path, &P);
+                        loadPath<N, CACHE>(a.fb, path, &P);
                         org = xyz(o4);
                         dir = xyz(d4);
                         tmax = d4.w;
@@ -1620,22 +1874,22 @@ k_tail(KArgs a) {
         h.b1 = h.b2 = 0.0f;
         constexpr bool kAlpha = NODES && !MULTI;
         if constexpr (kAlpha) P.rngUsed = P.rngUsed || sc.hasAlpha;
-        bool found = traceRay<false, STATS, kAlpha>(psc, org, dir, 0.0f, tmax, &h, lds, threadIdx.x, &tc, &P.rng);
+        bool found = traceRay<false, STATS, kAlpha, kLdsStack, false, TOP>(psc, org, dir, 0.0f, tmax, &h, lds, threadIdx.x, &tc, &P.rng);
         int4 ha = found ? make_int4(h.inst, h.geomInst, h.prim, 0) : make_int4(-1, -1, -1, 0);
         bool emitShadow, emitNext;
         float4 shOrg, shDir, shVal, nextOrg, nextDir;
-        shadeStep<N, NODES>(psc, depth + 1, maxLen, path, org, dir, ha, make_float2(h.b1, h.b2), P, cc, &emitShadow,
+        shadeStep<N, NODES, CACHE>(psc, depth + 1, maxLen, path, org, dir, ha, make_float2(h.b1, h.b2), P, cc, &emitShadow,
                      &shOrg, &shDir, &shVal, &emitNext, &nextOrg, &nextDir);
         if (emitShadow) {
             atomicAdd(&depthCounts[2 * depth + 1], 1u);
             TraceHit sh;
             float vis = 1.0f;
-            bool occluded = traceRay<true, STATS, kAlpha>(psc, xyz(shOrg), xyz(shDir), 0.0f, shDir.w, &sh, lds,
+            bool occluded = traceRay<true, STATS, kAlpha, kLdsStack, false, TOP>(psc, xyz(shOrg), xyz(shDir), 0.0f, shDir.w, &sh, lds,
                                                           threadIdx.x, &tcShadow, nullptr, &vis);
             if (!occluded) P.contrib += loadSpec<N>(shVal) * vis;
         }
         if (!emitNext) {
-            storePath<N>(a.fb, path, depth + 1, P, false);
+            storePath<N, CACHE>(a.fb, path, depth + 1, P, false);
             active = false;
             continue;
         }
@@ -2132,7 +2386,7 @@ __device__ __forceinline__ bool connectVisible(const DevScene &sc, const SurfPt 
     float tmax = 3.402823466e+38f;
     if (!light.atInfinity) tmax = (lo - so).length() * 0.9999f;
     TraceHit h;
-    return !traceRay<true, false, ALPHA>(sc, so, *dir, 0.0f, tmax, &h, lds, lane, nullptr, nullptr, vis);
+    return !traceRay<true, false, ALPHA, kLdsStack, false, false>(sc, so, *dir, 0.0f, tmax, &h, lds, lane, nullptr, nullptr, vis);
 }
 
 template <int N>
@@ -2226,7 +2480,7 @@ k_bptLight(BptArgs a) {
                 TraceHit h;
                 h.inst = -1;
                 h.b1 = h.b2 = 0.0f;
-                bool found = traceRay<false, false, NODES>(sc, rayOrg, rayDir, 0.0f, 3.402823466e+38f, &h, lds,
+                bool found = traceRay<false, false, NODES, kLdsStack, false, false>(sc, rayOrg, rayDir, 0.0f, 3.402823466e+38f, &h, lds,
                                                            threadIdx.x, nullptr, &rng);
                 V3 nextOrg, nextDir;
                 float woDirPDF = 0, woCosTerm = 0, woRevAreaPDF = 0;
@@ -2512,7 +2766,7 @@ k_bptEye(BptArgs a) {
             TraceHit h;
             h.inst = -1;
             h.b1 = h.b2 = 0.0f;
-            bool found = traceRay<false, false, NODES>(sc, rayOrg, rayDir, 0.0f, 3.402823466e+38f, &h, lds,
+            bool found = traceRay<false, false, NODES, kLdsStack, false, false>(sc, rayOrg, rayDir, 0.0f, 3.402823466e+38f, &h, lds,
                                                        threadIdx.x, nullptr, &rng);
             const Wls<N> wls = commonWls<N>(bp, single);
             if (GUIDES && pathLength == 1)
@@ -2865,7 +3119,7 @@ k_lightTrace(BptArgs a) {
                 TraceHit h;
                 h.inst = -1;
                 h.b1 = h.b2 = 0.0f;
-                if (!traceRay<false, false, NODES>(sc, rayOrg, rayDir, 0.0f, 3.402823466e+38f, &h, lds, threadIdx.x,
+                if (!traceRay<false, false, NODES, kLdsStack, false, false>(sc, rayOrg, rayDir, 0.0f, 3.402823466e+38f, &h, lds, threadIdx.x,
                                                    nullptr, &rng))
                     break;
                 SurfPt sp;
@@ -3130,10 +3384,17 @@ static hipError_t launchFrameT(const DevScene &sc, const FrameParams &fp, const 
         a.depth = wavefrontDepths;
         const uint32_t blocks = std::max(1u, std::min(blocksFor(n, kTraceBlock), fp.tailBlocks));
         t0(STAGE_TAIL);
+        const bool top = !NODES && a.sc.numTriangles >= kTopWalkTriangles;
         if (fp.traversalStats)
             hipLaunchKernelGGL((k_tail<N, true, false, NODES>), dim3(blocks), dim3(kTraceBlock), 0, s, a);
+        else if (fp.cacheMode != 0 && top)
+            hipLaunchKernelGGL((k_tail<N, false, false, NODES, true, !NODES>), dim3(blocks), dim3(kTraceBlock), 0, s, a);
+        else if (fp.cacheMode != 0)
+            hipLaunchKernelGGL((k_tail<N, false, false, NODES, true>), dim3(blocks), dim3(kTraceBlock), 0, s, a);
+        else if (top)
+            hipLaunchKernelGGL((k_tail<N, false, false, NODES, false, !NODES>), dim3(blocks), dim3(kTraceBlock), 0, s, a);
         else
-            hipLaunchKernelGGL((k_tail<N, false, false, NODES>), dim3(blocks), dim3(kTraceBlock), 0, s, a);
+            hipLaunchKernelGGL((k_tail<N, false, false, NODES, false>), dim3(blocks), dim3(kTraceBlock), 0, s, a);
         t1(STAGE_TAIL);
     }
     if (cache && fp.cacheMode == 2) {
@@ -3207,9 +3468,9 @@ static hipError_t launchBatchStepT(const BatchLaunch &b, hipStream_t s) {
         a.depth = wavefrontDepths;
         const uint32_t blocks = std::max(1u, std::min(blocksFor(n, kTraceBlock), b.fp.tailBlocks));
         if (b.nodePrograms)
-            hipLaunchKernelGGL((k_tail<N, false, true, true>), dim3(blocks), dim3(kTraceBlock), 0, s, a);
+            hipLaunchKernelGGL((k_tail<N, false, true, true, false, true>), dim3(blocks), dim3(kTraceBlock), 0, s, a);
         else
-            hipLaunchKernelGGL((k_tail<N, false, true, false>), dim3(blocks), dim3(kTraceBlock), 0, s, a);
+            hipLaunchKernelGGL((k_tail<N, false, true, false, false, true>), dim3(blocks), dim3(kTraceBlock), 0, s, a);
     }
     hipLaunchKernelGGL((k_accumulate<N, true>), dim3(blocksFor(n, 256)), dim3(256), 0, s, a);
     hipLaunchKernelGGL(k_frameEnd, dim3(1), dim3(64), 0, s, b.fb.counters, b.fp.maxPathLength, wavefrontDepths);

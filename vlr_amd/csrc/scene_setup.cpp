@@ -728,6 +728,7 @@ void buildSceneGPU(Context &ctx, const Scene &scene, bool spectral, SceneGPU *g)
     D.mengPoints = static_cast<const float *>(g->mengPoints.ptr);
     D.numInstances = static_cast<uint32_t>(insts.size());
     D.hasTlas = instBoxes.empty() ? 0 : 1;
+    D.numTriangles = static_cast<uint32_t>(std::min<uint64_t>(numTris, UINT32_MAX));
     cmfBins(D.cmfX, D.cmfY, D.cmfZ, &D.integralCMF);
     {
         ImmSpectrum white;
