@@ -82,7 +82,7 @@ constexpr int kShadowLds = kLdsStack * kTraceBlock;
 // Occupancy asked of the tail kernel.  It holds a path, a ray and a shading vertex; at 4 waves per SIMD
 // (128 VGPRs) it spilled 60 to 130 of them into its loops.  Measured at 4 / 3 waves: textured 720p
 // 3.95 / 3.49 ms (4 frames), cached 1080p 10.1 / 9.3 ms (8), Cornell box 256 x 256 4.78 / 4.63 ms (16),
-// icosphere grid 1080p 22.5 / 22.9 ms (8); at 2 waves the grid takes 26.3 ms.
+// icosphere grid 1080p 22.5 / 22.9 ms (8; the only one that loses); at 2 waves the grid takes 26.3 ms.
 constexpr int kTailWavesPerEU = 3;
 // Occupancy asked of the per-path LVC-BPT and light-tracing kernels.  Left to themselves they
 // take 130-230 VGPRs and run 2 waves per SIMD; with some registers spilled, more waves hide
@@ -482,6 +482,8 @@ __device__ __forceinline__ void spaceStep(TravState &st, const DevScene &sc, typ
 // programs (textured 720p 3.74 / 3.81 ms); they use walkLds.  So does the tail kernel where the walks
 // are too short for the top entry to matter (fewer than kTopWalkTriangles in the scene): the Cornell
 // box of 36 triangles at 256 x 256 takes 4.50 / 4.67 ms (16), 160 x 90 previews of it 262 / 269 us.
+// (Between that box and the 270 k triangles no scene was timed with both; 4096 are a few levels of inner
+// nodes.  Either walk gives the same bits.)
 constexpr uint32_t kTopWalkTriangles = 4096;
 template <bool ANY, bool STATS, bool ALPHA, int SD, bool CODES>
 __device__ __forceinline__ void walkTop(TravState &st, const DevScene &sc, int32_t *ldsWords, int lane,
