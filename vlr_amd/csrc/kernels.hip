@@ -805,14 +805,19 @@ __device__ __forceinline__ float envMapPDF(const DevScene &sc, float d0, float d
            continuousPDF(sc.distPool, sc.envRowBase + row * (2 * sc.envMapW + 1), sc.envMapW, d0);
 }
 
-// bilinear environment fetch, repeat wrapping in both axes (u and v lie in [0, 1], so the texels
-// left of and right of the sample are at most one past the edges)
+// bilinear environment fetch, repeat wrapping in both axes.  A direction's u and v lie in [0, 1]: its
+// left texel is at most one past the edges, which two selects wrap.  The texture coordinates of a mesh
+// that emits the environment texture lie anywhere; only they take the remainders.
 __device__ __forceinline__ float4 envFetch(const DevScene &sc, float u, float v) {
     float x = u * sc.envW - 0.5f, y = v * sc.envH - 0.5f;
     float fx0 = floorf(x), fy0 = floorf(y);
     float wx = x - fx0, wy = y - fy0;
     const int32_t W = static_cast<int32_t>(sc.envW), H = static_cast<int32_t>(sc.envH);
-    const int32_t x0 = min(max(static_cast<int32_t>(fx0), -1), W - 1), y0 = min(max(static_cast<int32_t>(fy0), -1), H - 1);
+    int32_t x0 = static_cast<int32_t>(fx0), y0 = static_cast<int32_t>(fy0);
+    if (static_cast<uint32_t>(x0) + 1u > sc.envW || static_cast<uint32_t>(y0) + 1u > sc.envH) {
+        x0 = ((x0 % W) + W) % W;
+        y0 = ((y0 % H) + H) % H;
+    }
     const int32_t xa = x0 < 0 ? W - 1 : x0, xb = x0 + 1 < W ? x0 + 1 : 0;
     const int32_t ya = y0 < 0 ? H - 1 : y0, yb = y0 + 1 < H ? y0 + 1 : 0;
     float4 t00 = sc.envTex[ya * W + xa], t10 = sc.envTex[ya * W + xb];
