@@ -66,3 +66,38 @@ def test_edge_rays_hit_what_brute_force_hits(torch_gpu, kind, scene, offset):
     np.testing.assert_array_equal(hits["inst"] >= 0, found)
     np.testing.assert_array_equal(hits["t"][found], ref["t"][found])
     np.testing.assert_array_equal(blocked, found)
+
+
+@pytest.mark.parametrize("lo,hi", [(-122, -100), (-100, -60), (60, 100), (100, 127)])
+@pytest.mark.parametrize("any_hit", [False, True])
+def test_directions_of_extreme_length(torch_gpu, lo, hi, any_hit):
+    """Scaling a direction by a power of two scales the hit's distance by its inverse and changes
+    nothing else, down to directions whose smaller components are denormal and up to those whose
+    reciprocals are.  The reference traces the directions scaled back, which is exact."""
+    desc = scenes.tessellated_cornell(3, 6000)
+    rays = edge_rays("", 4096 + 17, [-1.4, 0.1, -1.4], [1.4, 2.9, 1.4], 12)
+    rng = np.random.default_rng(13)
+    n = len(rays)
+    axis = rng.integers(0, 3, n)
+    d = rays["dir"].astype(np.float64)
+    # half of the rays leave a plane only slowly: two of the components are 1 and 3 to 100 times smaller
+    slow = rng.random(n) < 0.5
+    d[slow, axis[slow]] *= 10.0 ** -rng.uniform(0.5, 2, slow.sum())
+    exponent = rng.integers(lo, hi + 1, n)
+    rays["dir"] = np.ldexp(d, exponent[:, None]).astype(np.float32)
+    unit = rays.copy()
+    unit["dir"] = np.ldexp(rays["dir"].astype(np.float64), -exponent[:, None]).astype(np.float32)
+    with api.Context() as ctx:
+        bs = api.build_scene(ctx, desc)
+        hits = gpu_trace(torch_gpu, ctx, bs.scene, rays, any_hit=any_hit)
+    ref = ob.Scene(desc).trace_closest(unit, use_bvh=False)
+    found = ref["inst"] >= 0
+    assert found.mean() > 0.5
+    np.testing.assert_array_equal(hits["inst"] >= 0, found)
+    if not any_hit:
+        expected = np.ldexp(ref["t"].astype(np.float64), -exponent).astype(np.float32)
+        np.testing.assert_array_equal(hits["t"][found], expected[found])
+        same = found & (hits["prim"] == ref["prim"]) & (hits["geomInst"] == ref["geomInst"])
+        assert same.sum() > 0.99 * found.sum()      # the others tie on an edge of two triangles
+        np.testing.assert_array_equal(hits["b1"][same], ref["b1"][same])
+        np.testing.assert_array_equal(hits["b2"][same], ref["b2"][same])

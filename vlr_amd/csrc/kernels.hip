@@ -132,9 +132,11 @@ struct RayPre {
         Sx = rot1(d) / dkz;
         Sy = rot2(d) / dkz;
         Sz = 1.0f / dkz;
-        // Directions of a component below 2^-60 of the largest count as that: the planes' parameters
-        // stay finite, and no point of the ray moves by more than 2^-60 of its distance.
-        const float tiny = fmaxf(best * 8.6736174e-19f, 1.17549435e-38f);
+        // A component below 2^-60 of the largest counts as that, by which no point of the ray moves by
+        // more than 2^-60 of its distance.  Where even that is too small to have a finite reciprocal, the
+        // axis's planes come out as NaN or as infinities that exclude nothing, and the axis culls no box.
+        // (A zero direction hits no triangle; finite reciprocals keep it out of most boxes.)
+        const float tiny = best > 0.0f ? best * 8.6736174e-19f : 1.17549435e-38f;
         inv.x = __builtin_amdgcn_rcpf(copysignf(fmaxf(adx, tiny), d.x));
         inv.y = __builtin_amdgcn_rcpf(copysignf(fmaxf(ady, tiny), d.y));
         inv.z = __builtin_amdgcn_rcpf(copysignf(fmaxf(adz, tiny), d.z));
@@ -3273,13 +3275,25 @@ __global__ void __launch_bounds__(kTraceBlock) k_traceRays(DevScene sc, const Ra
     RayIn r = rays[i];
     TraceHit h;
     h.inst = -1; h.geomInst = -1; h.prim = -1; h.t = 0; h.b1 = 0; h.b2 = 0;
-    bool f = traceRay<ANY>(sc, V3(r.org[0], r.org[1], r.org[2]), V3(r.dir[0], r.dir[1], r.dir[2]), r.tmin, r.tmax,
-                           &h, lds, threadIdx.x);
+    V3 dir(r.dir[0], r.dir[1], r.dir[2]);
+    // A caller's direction may have any length.  The walk needs finite, normal reciprocals of its larger
+    // components, so a length far from 1 is brought near it by a power of two, which scales the hit's
+    // distance by the inverse and leaves everything else as it is.
+    const float longest = fmaxf(fabsf(dir.x), fmaxf(fabsf(dir.y), fabsf(dir.z)));
+    int e = 0;
+    if (longest < 0x1p-60f || longest > 0x1p60f) e = __builtin_amdgcn_frexp_expf(longest);   // 0 for 0 and infinity
+    if (e != 0) dir = V3(ldexpf(dir.x, -e), ldexpf(dir.y, -e), ldexpf(dir.z, -e));
+    auto scaled = [&](float t) {   // a positive limit stays one
+        const float s = ldexpf(t, e);
+        return t > 0.0f ? fmaxf(s, 0x1p-149f) : s;
+    };
+    bool f = traceRay<ANY>(sc, V3(r.org[0], r.org[1], r.org[2]), dir, scaled(r.tmin), scaled(r.tmax), &h, lds,
+                           threadIdx.x);
     HitOut o;
     o.inst = f ? h.inst : -1;
     o.geomInst = f ? h.geomInst : -1;
     o.prim = f ? h.prim : -1;
-    o.t = f ? h.t : 0.0f;
+    o.t = f ? ldexpf(h.t, -e) : 0.0f;
     o.b1 = f ? h.b1 : 0.0f;
     o.b2 = f ? h.b2 : 0.0f;
     hits[i] = o;
