@@ -25,7 +25,19 @@ def moved(desc, offset):
     return desc
 
 
-def edge_rays(kind, n, lo, hi, seed):
+def vertex_coordinates(desc):
+    """World-space vertex coordinates per axis, by the float32 transform of the library."""
+    out = [[], [], []]
+    for inst in desc.instances:
+        m = inst.transform.reshape(4, 4, order="F").astype(np.float32)
+        for k in inst.meshes:
+            p = desc.meshes[k].vertices[:, 0:3]
+            for a in range(3):
+                out[a].append(m[a, 0] * p[:, 0] + m[a, 1] * p[:, 1] + m[a, 2] * p[:, 2] + m[a, 3])
+    return [np.unique(np.concatenate(c)) for c in out]
+
+
+def edge_rays(kind, n, lo, hi, seed, coords=None):
     rng = np.random.default_rng(seed)
     rays = np.zeros(n, api.RAY_DTYPE)
     d = rng.normal(size=(n, 3))
@@ -42,8 +54,10 @@ def edge_rays(kind, n, lo, hi, seed):
         d[np.arange(n), axis] *= 10.0 ** -rng.uniform(6, 44, n)
     elif kind == "unnormalised":
         d *= 10.0 ** rng.uniform(-12, 12, (n, 1))
-    elif kind == "on planes":         # origins on the coordinates of the boxes' corners
-        o[np.arange(n), axis] = rng.choice([lo[1], hi[1], 0.0, 0.6, 1.2, 2.99], n)
+    elif kind == "on planes":         # origins on the planes of vertices, which the boxes' faces lie in
+        for a in range(3):
+            inside = coords[a][(coords[a] >= lo[a]) & (coords[a] <= hi[a])]
+            o[axis == a, a] = rng.choice(inside, (axis == a).sum())
     rays["org"], rays["dir"], rays["tmax"] = o.astype(np.float32), d.astype(np.float32), INF
     return rays
 
@@ -54,7 +68,10 @@ def test_edge_rays_hit_what_brute_force_hits(torch_gpu, kind, scene, offset):
     desc = scenes.cornell_box() if scene == "cornell" else scenes.tessellated_cornell(3, 6000)
     desc = moved(desc, (offset, -offset, 0.5 * offset))
     c = np.array([offset, -offset, 0.5 * offset])
-    rays = edge_rays(kind, 4096 + 17, c + [-1.6, -0.1, -1.6], c + [1.6, 3.1, 1.6], 11)
+    coords = vertex_coordinates(desc)
+    rays = edge_rays(kind, 4096 + 17, c + [-1.6, -0.1, -1.6], c + [1.6, 3.1, 1.6], 11, coords)
+    if kind == "on planes":
+        assert np.all(np.any([np.isin(rays["org"][:, a], coords[a]) for a in range(3)], axis=0))
     with api.Context() as ctx:
         bs = api.build_scene(ctx, desc)
         hits = gpu_trace(torch_gpu, ctx, bs.scene, rays)
@@ -62,7 +79,7 @@ def test_edge_rays_hit_what_brute_force_hits(torch_gpu, kind, scene, offset):
     ref = ob.Scene(desc).trace_closest(rays, use_bvh=False)
     found = ref["inst"] >= 0
     print(kind, scene, offset, "hits", found.mean())
-    assert found.any()
+    assert found.mean() > 0.5
     np.testing.assert_array_equal(hits["inst"] >= 0, found)
     np.testing.assert_array_equal(hits["t"][found], ref["t"][found])
     np.testing.assert_array_equal(blocked, found)
