@@ -43,9 +43,11 @@ constexpr uint32_t kBvhMaxPrims = 1u << 28;  // leaf code limit (first << kLeafS
 
 // Traversal node stack per ray: kLdsStack entries in LDS, kScratchStack more in scratch.  A
 // visit of an inner 4-wide node pushes at most 3 entries and descends one level; entering an
-// instance pushes one marker.  A two-level walk therefore never holds more than
-// travStackBound(TLAS depth, deepest BLAS depth) entries, and scene set-up refuses trees whose
-// bound exceeds the capacity, so no entry is ever lost.
+// instance pushes one marker (walkTop) or notes the stack's height in its place (walkLds).  A two-level
+// walk therefore never holds more than travStackBound(TLAS depth, deepest BLAS depth) entries, and
+// scene set-up refuses trees whose bound exceeds the capacity, so no entry is ever lost.  (walkTop
+// also stacks a marker below the first entry and loads one place below that when it ends; its scratch
+// part is two entries longer.)
 constexpr int kLdsStack = 16;
 constexpr int kScratchStack = 64;
 constexpr uint32_t kTravStackCapacity = kLdsStack + kScratchStack;
@@ -69,8 +71,9 @@ __host__ __device__ inline int bvhBin(float c, float clo, float ext) {
 }
 
 // One quantised node: per axis the grid step is the power of two 2^k with 255 * 2^k >= the
-// node extent; each child plane is rounded outwards and checked with the decoding arithmetic
-// the traversal uses (origin + float(q) * step: an exact product and one rounded sum).
+// node extent; each child plane is rounded outwards and checked as decoded (origin + float(q) * step:
+// an exact product and one rounded sum).  The traversal takes a plane's ray parameter by one
+// multiply-add from q, with a bound on its rounding that counts this one in.
 __host__ __device__ inline BVH4QNode quantizeBvh4Node(const BVH4Node &f) {
     BVH4QNode q;
     for (int a = 0; a < 3; ++a) {

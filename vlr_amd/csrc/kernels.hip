@@ -10,8 +10,8 @@
 //                 k_shade      hit/miss programs (path_tracing.cu:133-337): implicit emission
 //                              with MIS, Russian roulette, next-event estimation (builds a
 //                              shadow ray, light_transport_common.h:147-192), BSDF sampling;
-//                              appends the next ray and the shadow ray with wave-aggregated
-//                              atomics
+//                              appends the next ray and the shadow ray, one atomic per block
+//                              and queue
 //                 k_shadow     any-hit traversal, adds the NEE contribution if unoccluded
 //   k_accumulate  Kahan accumulation (path_tracing.cu:119-127)
 //   k_convert     XYZ -> Rec.709 output (post_process.cu:93-163)
@@ -102,11 +102,13 @@ constexpr int32_t kSentinel = INT32_MIN;
 // plane, with the node's six constants computed once for its four children, where decoding the
 // plane first (q * s, + o, - org, * inv) takes five operations.  The sign of the direction selects
 // which of the two planes is the near one for all four children at once, in place of a minimum and
-// a maximum per child and axis.  The traversal is bound by VALU issue (k_tail: 0.62 of one
-// instruction per CU and cycle at 19 % of its lanes), so operations count: against decoded planes,
-// generic stack pointers (flat accesses) and per-child branches, a 256 x 256 Cornell frame went from
-// 0.52 to 0.30 ms, the 1080p icosphere grid's from 3.9 to 3.4 ms, 2^21 incoherent closest-hit rays
-// in that grid from 2.14 to 1.80 ms.
+// a maximum per child and axis.  A wave walks one dependent chain (fetch a node, test its planes, fetch
+// the child) with few lanes active (22 % in k_tail on the icosphere grid) and little else to issue: a
+// SIMD issues a VALU instruction on 15 % of its cycles there, on 4 % in a 256 x 256 Cornell frame.  So
+// the operations between two fetches count by their latency: against decoded planes, generic stack
+// pointers (flat accesses) and per-child branches, a 256 x 256 Cornell frame went from 0.52 to
+// 0.30 ms, the 1080p icosphere grid's from 3.9 to 3.4 ms, 2^21 incoherent closest-hit rays in that grid
+// from 2.14 to 1.80 ms.
 //   The constants cancel (o - org against q * s), so their rounding is bounded absolutely.  With
 // u = 2^-24, a = s * inv, b = fma(o, inv, -org * inv) and M = |org inv| + |b| + 256 |a|, a computed
 // plane parameter is off by: the plane as stored (the builder's check rounds o + q * s once), at
@@ -211,7 +213,7 @@ struct TravCount {
 typedef int32_t StackPair __attribute__((ext_vector_type(2)));   // node code, entry distance
 
 // Traversal state: one ray's walk through the two-level BVH.  The node stack lives in LDS
-// (kLdsStack entries per lane) with an overflow area in scratch, its top entry in registers.
+// (kLdsStack entries per lane) with an overflow area in scratch; walkTop has its top entry in registers.
 constexpr int32_t kTravDone = INT32_MIN + 1;
 struct TravState {
     V3 org, dir;                  // the world-space ray
@@ -253,7 +255,7 @@ __device__ __forceinline__ void travBegin(TravState &st, const DevScene &sc, con
     st.vis = 1.0f;
 }
 
-// Stack entries below the top: SD per lane in LDS, (code, entry distance) pairs of which an any-hit
+// walkTop's stack entries below the top: SD per lane in LDS, (code, entry distance) pairs of which an any-hit
 // ray uses the codes, and the others in scratch.  A lane's entries have the same places for both
 // kinds of rays, because the waves of a block run the two at the same time.  CODES: places for codes
 // only, in a kernel that traces nothing but any-hit rays.
@@ -478,14 +480,18 @@ __device__ __forceinline__ void spaceStep(TravState &st, const DevScene &sc, typ
 // walkTop keeps the stack's top entry in registers, so that the node after a miss is known before
 // the LDS is read, and loads a leaf's next triangle while it tests one; walkLds keeps neither.
 // Measured, walkLds / walkTop: 2^21 incoherent rays in the icosphere grid 1.77 / 1.40 ms, its 1080p
-// frames 26.3 / 22.8 ms (8), 270 k triangles at 641 x 427 3.86 / 3.45 ms (4), a batch of 24 jobs
-// 33.9 / 33.0 ms.  The kernels that spill in any case lose by the registers more than they gain:
-// LVC-BPT 720p 6.64 / 6.93 ms, light tracing 720p 3.46 / 3.60 ms, and the tail kernel with node
-// programs (textured 720p 3.74 / 3.81 ms); they use walkLds.  So does the tail kernel where the walks
-// are too short for the top entry to matter (fewer than kTopWalkTriangles in the scene): the Cornell
-// box of 36 triangles at 256 x 256 takes 4.50 / 4.67 ms (16), 160 x 90 previews of it 262 / 269 us.
-// (Between that box and the 270 k triangles no scene was timed with both; 4096 are a few levels of inner
-// nodes.  Either walk gives the same bits.)
+// frames 26.3 / 22.8 ms (8), 270 k triangles at 641 x 427 3.86 / 3.45 ms (4).  The kernels that spill in
+// any case lose by the registers more than they gain: LVC-BPT 720p 6.64 / 6.93 ms, light tracing 720p
+// 3.46 / 3.60 ms, and single images with node programs (textured 720p 3.74 / 3.81 ms); they use
+// walkLds.  So does the tail kernel where the walks are too short for the top entry to matter, which it
+// tells by the scene's triangles (720p, 4 frames, RGB, every depth in the tail kernel):
+//   36 triangles 2.96 / 3.02 ms, 1,316 3.27 / 3.30, 3,876 3.80 / 3.75, 10,276 4.40 / 4.26, 50 k 4.93 / 4.64;
+//   256 x 256 and 36 triangles, 16 frames, 4.50 / 4.58 ms.
+// The triangles of a mesh count once however many instances share it, so the grid with one sphere mesh
+// in all instances takes walkLds though its walks are long: 64 instances 5.64 / 5.17 ms, 576 instances
+// 5.99 / 5.37 ms.  The depths of the trees would tell such scenes.  Batches, whose jobs share a
+// launch, always use walkTop: 24 jobs of 10 k to 60 k triangles 33.9 / 33.0 ms, 8 Cornell boxes
+// 6.07 / 6.15 ms, 8 boxes with node programs 7.59 / 7.63 ms (RGB) and 8.94 / 8.83 ms (spectral).
 constexpr uint32_t kTopWalkTriangles = 4096;
 template <bool ANY, bool STATS, bool ALPHA, int SD, bool CODES>
 __device__ __forceinline__ void walkTop(TravState &st, const DevScene &sc, int32_t *ldsWords, int lane,
@@ -3402,9 +3408,9 @@ static hipError_t launchFrameT(const DevScene &sc, const FrameParams &fp, const 
         t0(STAGE_SHADE);
         if (fp.sortShade) hipLaunchKernelGGL(k_sortScatter, dim3(blocksFor(n, 256)), dim3(256), 0, s, a);
         if (guides && d == 0)
-            hipLaunchKernelGGL((k_shade<N, false, NODES, true>), dim3(blocksFor(n, 256)), dim3(256), 0, s, a);
+            hipLaunchKernelGGL((k_shade<N, false, NODES, true>), dim3(blocksFor(n, kShadeBlock)), dim3(kShadeBlock), 0, s, a);
         else
-            hipLaunchKernelGGL((k_shade<N, false, NODES>), dim3(blocksFor(n, 256)), dim3(256), 0, s, a);
+            hipLaunchKernelGGL((k_shade<N, false, NODES>), dim3(blocksFor(n, kShadeBlock)), dim3(kShadeBlock), 0, s, a);
         t1(STAGE_SHADE);
         t0(STAGE_SHADOW);
         if (sc.hasAlpha)
@@ -3498,9 +3504,9 @@ static hipError_t launchBatchStepT(const BatchLaunch &b, hipStream_t s) {
         a.depth = d;
         hipLaunchKernelGGL((k_intersect<false, true>), dim3(blocksFor(n, kTraceBlock)), dim3(kTraceBlock), 0, s, a);
         if (b.nodePrograms)
-            hipLaunchKernelGGL((k_shade<N, true, true>), dim3(blocksFor(n, 256)), dim3(256), 0, s, a);
+            hipLaunchKernelGGL((k_shade<N, true, true>), dim3(blocksFor(n, kShadeBlock)), dim3(kShadeBlock), 0, s, a);
         else
-            hipLaunchKernelGGL((k_shade<N, true, false>), dim3(blocksFor(n, 256)), dim3(256), 0, s, a);
+            hipLaunchKernelGGL((k_shade<N, true, false>), dim3(blocksFor(n, kShadeBlock)), dim3(kShadeBlock), 0, s, a);
         hipLaunchKernelGGL((k_shadow<false, true>), dim3(blocksFor(n, kTraceBlock)), dim3(kTraceBlock), 0, s, a);
     }
     if (wavefrontDepths < numDepths) {

@@ -59,7 +59,7 @@ struct CacheBuffers {
     uint32_t* trainAfterStamp;     // the path went on to a next vertex (trainContrib is set)
 };
 
-constexpr uint32_t kDefaultTailBlocks = 2048;   // 8 blocks of 128 per CU
+constexpr uint32_t kDefaultTailBlocks = 2048;   // 8 blocks of 128 per CU, 6 of them resident at 3 waves per SIMD
 
 // Frame-schedule autotuner.  The image does not depend on the schedule, so candidates are
 // timed on real frames: first the wavefront depth (tail grid fixed), then the tail grid at

@@ -495,8 +495,8 @@ __device__ __forceinline__ Bsdf<N> setupBsdf(const DevScene &sc, const DevMateri
     if (spectra > 1) b.c1 = materialSpectrum<N>(sc, m, 1, o, bins);
     if (spectra > 2) b.c2 = materialSpectrum<N>(sc, m, 2, o, bins);
     // microfacet types (materials.cu:1226-1236, 1516-1536): alphas and rotation, derived on the host
-    // unless a node supplies the parameters.  (No switch with these two types sharing a case: its
-    // gfx950 code lost the first of the three for one of them.)
+    // unless a node supplies the parameters.  (A switch in which the two types shared a case gave NaN for
+    // microfacet scattering in RGB; whether that code or its compilation was at fault was not found out.)
     const bool micro = type == MAT_MICROFACET_REFLECTION || type == MAT_MICROFACET_SCATTERING;
     float ax = m.scalars[0], ay = m.scalars[1], rotation = m.scalars[2];
     if (micro && (o.has & 8u)) ggxParams(o.vec[0], &ax, &ay, &rotation);
