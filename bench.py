@@ -105,14 +105,16 @@ def cpu_model():
     return platform.processor()
 
 
-def read_traffic(kernel):
-    """HBM bytes per launch of `kernel` on this workload, from the committed counter summary
-    (rocprofv3 FETCH_SIZE + WRITE_SIZE, scaled by a copy kernel of known size), if present."""
+def read_traffic(kernel, wavefront_depth):
+    """HBM bytes per launch of `kernel` on this workload at this wavefront depth, from the
+    committed counter summary (rocprofv3 FETCH_SIZE + WRITE_SIZE, scaled by a copy kernel of known
+    size); None where it holds no run at that depth."""
     path = os.path.join(ROOT, "profiles", f"{kernel}_icosphere_grid_1080p_traffic.json")
     if not os.path.exists(path):
         return None
     with open(path) as f:
-        return float(json.load(f)["hbm_bytes_per_launch"])
+        run = json.load(f)["wavefront_depth"].get(str(wavefront_depth))
+    return None if run is None else float(run["hbm_bytes_per_launch"])
 
 
 def cpu_threads():
@@ -673,7 +675,7 @@ def main():
     per_launch_bytes = total_bytes / max(1, launches)
     mean_launch_s = ms / 1e3 / max(1, launches)
     achieved = per_launch_bytes / mean_launch_s / 1e9
-    traffic = read_traffic(dominant)
+    traffic = read_traffic(dominant, sched_wd)
 
     out = {
         "metric": METRIC,
@@ -706,7 +708,8 @@ def main():
                      "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
                      "traffic_source": None if traffic is None else
                      f"profiles/{dominant}_icosphere_grid_1080p_traffic.json (rocprofv3 FETCH_SIZE + WRITE_SIZE "
-                     f"of this workload, scaled by a copy of known size; not measured in this run)",
+                     f"of this workload at this wavefront depth, scaled by a copy of known size; not measured in "
+                     f"this run)",
                      "algorithmic_bytes_per_launch": per_launch_bytes, "mean_launch_ms": mean_launch_s * 1e3},
         "image_mean_rgb": [float(x) for x in img[..., :3].reshape(-1, 3).mean(axis=0)],
         "setup_s": setup_s,
